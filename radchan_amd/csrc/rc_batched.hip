@@ -14,13 +14,13 @@
  * The main loop generates rays in bulk (all 64 lanes set up one ray each),
  * refills idle lanes from the queue once enough of them are idle (at the
  * top of the iteration, and in refill mode 1 also between its steps), and
- * advances every lane by a few steps (march_core_bulk, the loop body of
- * march_ray; a ray that meets a black wall takes the wall's emission on
- * its next step, through that step's own table lookup).  Rays keep their
+ * advances every live lane by a few steps (bulk_step in rc_bulk.h, the loop
+ * body of march_ray; a ray that meets a black wall takes the wall's emission
+ * on its next step, through that step's own table lookup).  Rays keep their
  * (sorted) order of dispatch, so neighbouring lanes march neighbouring
- * bands.  Each finished ray adds its FP32 tally to
- * its unit's FP64 total in an LDS slot; a slot's total goes to HBM when the
- * slot is reused.  When no unit is left the wavefront drains its last rays
+ * bands.  A ray that has ended waits in its lane until the next refill, when
+ * all of them add their FP32 tallies to their units' FP64 totals in LDS
+ * slots; a slot's total goes to HBM when the slot is reused.  When no unit is left the wavefront drains its last rays
  * (look-ahead march, then a whole-wavefront march of the longest ones).
  * Every per-ray result is bit-identical to the plain path and the CPU
  * oracle; only the summation order of the FP64 totals differs.
@@ -36,6 +36,7 @@
 #include "rc_device.h"
 #include "rc_internal.h"
 #include "rc_kernels.h"
+#include "rc_bulk.h"
 #include "rc_march.h"
 #include "rc_radix.h"
 
@@ -238,32 +239,42 @@ __device__ __forceinline__ void q_put(uint32_t *q, int qs, float sx, float sy, f
                         ((uint32_t)unit & 0xFFFFu) | ((uint32_t)h << 16), (uint32_t)tid);
 }
 
-template <bool SURF>
-__device__ __forceinline__ void q_get(const uint32_t *q, int qs, const Slots &sl, const DevCommon &cm,
-                                      const DevSnap &sn, Ray &r, En &e, int &unit, int &tid, int &h) {
+/* the queued ray `qs` taken by a lane: its state at its start cell on the
+ * finest level (dim), `wstep` the wavefront's step count */
+template <bool SURF, int TM>
+__device__ __forceinline__ void q_get(const uint32_t *q, int qs, const Slots &sl, const DevSnap &sn, const BulkDim &dim,
+                                      uint32_t st, int wstep, int maxs, BulkRay &b) {
     const uint4 *rec = reinterpret_cast<const uint4 *>(q + qs * QREC);
-    const uint4 a = rec[0], b = rec[1], c = rec[2];
-    r.sx = __uint_as_float(a.x);
-    r.sy = __uint_as_float(a.y);
-    r.sz = __uint_as_float(a.z);
-    r.isx = __uint_as_float(a.w);
-    r.isy = __uint_as_float(b.x);
-    r.isz = __uint_as_float(b.y);
-    r.f0 = r.sx < 0.f; r.f1 = r.sy < 0.f; r.f2 = r.sz < 0.f;
-    r.tra = 1.0f;
-    e.W = __uint_as_float(b.z);
-    e.Bi = __uint_as_float(b.w);
-    e.invBi = __uint_as_float(c.x);
-    e.row = c.y & 0xFFFFu;
-    e.rank = (int)(c.y >> 16);
-    unit = (int)(c.z & 0xFFFFu);
-    h = (int)(c.z >> 16);
-    tid = (int)c.w;
-    const uint4 *pr = reinterpret_cast<const uint4 *>(&sl.pl[unit & (NSLOT - 1)]);
+    const uint4 ra = rec[0], rb = rec[1], rc = rec[2];
+    b.sx = __uint_as_float(ra.x);
+    b.sy = __uint_as_float(ra.y);
+    b.sz = __uint_as_float(ra.z);
+    b.isx = __uint_as_float(ra.w);
+    b.isy = __uint_as_float(rb.x);
+    b.isz = __uint_as_float(rb.y);
+    b.W = __uint_as_float(rb.z);
+    b.Bi = __uint_as_float(rb.w);
+    b.invBi = __uint_as_float(rc.x);
+    /* byte offset of the table row: below 65536 (nT + 13) 8 */
+    b.rowb = __umul24(rc.y & 0xFFFFu, st * (TM == TAB_BF16 ? 4u : 8u));
+    b.rankb = TM == TAB_BF16 ? __umul24(rc.y >> 16, st * 16u) : 0u;
+    b.uh = rc.z;
+    b.tid = (int)rc.w;
+    const uint4 *pr = reinterpret_cast<const uint4 *>(&sl.pl[rc.z & (NSLOT - 1)]);
     const uint4 p0 = pr[0], p1 = pr[1];
+    Ray r;
     r.ic = (int)p0.x; r.jc = (int)p0.y; r.kc = (int)p0.z;
     r.xp = __uint_as_float(p0.w); r.yp = __uint_as_float(p1.x); r.zp = __uint_as_float(p1.y);
-    if (SURF) surface_adjust(sn, r);
+    if (SURF) {
+        r.f0 = b.sx < 0.f; r.f1 = b.sy < 0.f; r.f2 = b.sz < 0.f;
+        surface_adjust(sn, r);
+    }
+    b.xp = r.xp; b.yp = r.yp; b.zp = r.zp;
+    b.tra = 1.0f;
+    b.dacc = 0.f;
+    b.kt = KT_NONE;
+    b.cap = wstep + bulk_cap(maxs);
+    bulk_place(dim, r.ic, r.jc, r.kc, b);
 }
 
 /* the distance from unit number u (16 bits, as the ray records hold it)
@@ -375,38 +386,25 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
     int part = (int)(blockIdx.x % QPARTS), ptries = 0;   /* workgroups are dealt round-robin over the XCDs */
     Unit U{};
 
-    /* lane state; an idle lane keeps in-range values, since the march step
-     * runs in every lane */
-    bool active = false;
-    Ray r;
-    r.ic = r.jc = r.kc = 1;
-    r.f0 = r.f1 = r.f2 = 0;
-    r.xp = r.yp = r.zp = 0.f;
-    r.sx = r.sy = r.sz = 1.f;
-    r.isx = r.isy = r.isz = 1.f;
-    r.tra = 0.f;
-    En e;
-    e.row = 0u;
-    e.rank = 0;
-    e.W = 0.f;
-    e.Bi = 1.f;
-    e.invBi = 1.f;
-    float dacc = 0.f;
-    int runit = 0, rtid = 0, rh = 0, lev = 0, counter = 0;
-    int kt = -1;                  /* the lane's cached table pair (t, values) */
-    KbRaw kc;
-    kc.q = make_float4(0.f, 0.f, 0.f, 0.f);
-    kc.w = 0u;
-    kc.a = 0.f;
-    int wall = 0;                 /* the ray waits at a black wall, entry widx of the level's positions */
-    uint32_t widx = 0u;
-    LaneLevel ll{};               /* multigrid: the level of the lane's ray */
-    CellWalk cw;                  /* the ray's linear cell index and its steps along y and z */
-    cw.cell = 0u;
-    cw.dcy = cw.dcz = 0;
-    int nsteps = 0, nrays = 0;
-    int bsub = 0;                 /* bulk march sub-steps of the wavefront (every lane steps) */
+    /* lane state: actm, the lanes with a live ray; pend, those whose ray has
+     * ended since the last pick-up and is still to be tallied; wstep, the
+     * steps the wavefront has made */
+    unsigned long long actm = 0ull, pend = 0ull;
+    int wstep = 0;
+    BulkRay b{};
+    const uint32_t st = (uint32_t)tab_stride(cm.nT);
+    const bool open = cm.bd[FB] == 5 || cm.bd[FT] == 5;
+    int nsteps = 0;
+    long nrays = 0;               /* rays ended (wavefront total) */
+    int bsub = 0;                 /* bulk march sub-steps of the wavefront */
     int64_t bsteps = 0;           /* steps of live rays in the bulk march (wavefront total) */
+    /* the tallies of the rays that have ended */
+    auto finish_pending = [&]() {
+        if (lane_in(pend))
+            finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), bulk_dump(b, tol), de);
+        nrays += __popcll(pend);
+        pend = 0ull;
+    };
 
     for (;;) {
         /* (a) once the current unit is fully generated, take the next unit
@@ -501,8 +499,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                 }
             }
         }
-        const unsigned long long live = __ballot(active);
-        if (cur_h >= P && nxt >= 0 && (nxt_s == snap || (live == 0ull && qcount == 0)) &&
+        if (cur_h >= P && nxt >= 0 && (nxt_s == snap || (actm == 0ull && qcount == 0)) &&
             (qcount == 0 || unit_age(seq, uni((int)(rq[qhead * QREC + 10] & 0xFFFFu))) < NSLOT)) {
             /* (b) start the prepared unit (a new snapshot only once every
              * lane and the queue are empty; never over the slot of a ray
@@ -588,94 +585,89 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                 qcount += ng;
                 cur_h += ng;
             }
-            /* (d) idle lanes take queued rays, once `threshold` lanes
-             * are idle (or the queue holds fewer rays) */
-            auto take_rays = [&](unsigned long long idle) {
+            /* the level(s) of the current snapshot: sizes, x faces and
+             * positions (single grid: level 0's own arrays; several levels:
+             * those of all levels, a lane's level offset from them) */
+            const bool have = snap >= 0;
+            const DevSnap &sn0 = snaps[have ? snap : 0];
+            const SnapView sv = snap_view(&sn0);
+            const DevLevel l0 = level_view(&sn0.lev[0]);
+            const BulkDim d0{l0.im, l0.jm, l0.km, MULTI ? (uint32_t)l0.xoff : 0u, MULTI ? (uint32_t)l0.poff : 0u};
+            const float *xb = MULTI ? sv.xu_all : l0.xu;
+            const float *pb = MULTI ? sv.P_all : l0.P;
+            /* (d) once `threshold` lanes are idle (or the queue holds fewer
+             * rays), the rays that have ended are tallied and idle lanes take
+             * queued rays */
+            auto take_rays = [&]() {
+                const unsigned long long idle = ~actm;
                 const int nidle = __popcll(idle);
                 if (qcount > 0 && nidle >= min(threshold, qcount)) {
+                    finish_pending();
                     const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
                     const int npop = min(nidle, qcount);
-                    if (!active && rank < npop) {
-                        q_get<SURF>(rq, qwrap(qhead + rank), sl, cm, snaps[snap], r, e, runit, rtid, rh);
-                        active = true;
-                        dacc = 0.f;
-                        lev = 0;
-                        counter = 0;
-                        kt = -1;
-                        wall = 0;
+                    const bool take = lane_in(idle) && rank < npop;
+                    if (take) {
+                        q_get<SURF, TM>(rq, qwrap(qhead + rank), sl, sn0, d0, st, wstep, l0.maxs, b);
                         if (MULTI) {
-                            ll = lane_level(llev[0]);
-                            cell_walk_setup(ll, r, cw);
-                        } else {
-                            cell_walk_setup(level_view(&snaps[snap].lev[0]), r, cw);
+                            b.lev = 0;
+                            b.dy = l0.dy;
+                            b.dz = l0.dz;
                         }
+                        bulk_load(xb, pb, b);
                     }
+                    actm |= __ballot(take);
                     qhead = qwrap(qhead + npop);
                     qcount -= npop;
                 }
             };
-            take_rays(~live);
+            take_rays();
             const bool drained = qdone && nxt < 0 && cur_h >= P && qcount == 0;
-            if (drained && (__ballot(active) == 0ull || xfit)) break;   /* to the drain (f) */
-            if (__ballot(active) != 0ull) {
-                /* (e) march steps of every active lane; the snapshot's
-                 * fields (and the level, single grid) are wavefront-uniform
-                 * values, a lane's level is held in its registers
-                 * (multigrid: ll, set at pick-up and at each coarsening) */
-                const SnapView sv = snap_view(snaps + snap);
-                DevLevel l0;
-                if (!MULTI) l0 = level_view(&snaps[snap].lev[0]);
-                const float *xb = MULTI ? sv.xu_all : l0.xu;
-                const float *pb = MULTI ? sv.P_all : l0.P;
-                const uint32_t xmax = MULTI ? (uint32_t)(sv.nxu - 1) : (uint32_t)l0.im;
-                const uint32_t pmax = MULTI ? (uint32_t)(sv.npos - 1)
-                                            : (uint32_t)(level_pos_count(l0.im, l0.jm, l0.km) - 1);
-                /* spi march steps.  Every active lane holds a live ray under
-                 * its level's step cap: a ray is finished (or coarsened)
-                 * right after the step that ends it.  Idle lanes step too, on
-                 * stale state that the next pick-up overwrites; the step
-                 * bounds its loads. */
+            if (drained && (actm == 0ull || xfit)) break;   /* to the drain (f) */
+            if (actm != 0ull) {
+                /* (e) spi march steps of every live lane */
                 bsub += spi;
-                auto substep = [&](const auto &L, uint32_t xo, uint32_t po) {
-                    /* a wall step is no march step of the reference (its
-                     * tally belongs to the step that crossed the face): it
-                     * neither counts nor meets the step cap */
-                    const bool ws = wall != 0;
-                    const bool out = march_core_bulk<TM>(cm, sv, L, xb, xo, xmax, pb, po, pmax, r, e, tol, dacc, kt,
-                                                         kc, ws, widx, cw);
-                    boundary_defer(cm, L, r, active && out, wall, widx, cw);
-                    counter += 1;           /* a wall step ends the ray: its count is never read */
-                    bsteps += __popcll(__ballot(active && !ws));
-                    const bool alive = r.tra > tol;
-                    const bool done = active && (!alive || (counter >= L.maxs && wall == 0));
-                    const bool fin = done && (!MULTI || !alive || lev == cm.grid_num - 1);
-                    const bool crs = MULTI && done && !fin;
-                    if (fin) {
-                        finish_ray(cm, sl, seq, runit, rtid, rh, dacc, de);
-                        nrays += 1;
-                        active = false;
-                        wall = 0;
-                    }
-                    if (crs) {
-                        /* coarsen the indices for the next grid level (:215-223) */
-                        const DevLevel &Lc = llev[lev];
-                        r.ic = coarsen(r.ic, Lc.cr[0], Lc.cmul[0]);
-                        r.jc = coarsen(r.jc, Lc.cr[1], Lc.cmul[1]);
-                        r.kc = coarsen(r.kc, Lc.cr[2], Lc.cmul[2]);
-                        ll = lane_level(llev[lev + 1]);
-                        cell_walk_setup(ll, r, cw);
-                        lev += 1;
-                        counter = 0;
-                    }
-                };
 #pragma unroll 1
                 for (int q = 0; q < spi; ++q) {
                     /* refill between the steps too: a lane whose ray ended
                      * idles for less of the iteration */
-                    if (cm.refill && q > 0) take_rays(~__ballot(active));
-                    if (MULTI) substep(ll, ll.xoff, ll.poff);
-                    else substep(l0, 0u, 0u);
+                    if (cm.refill && q > 0) take_rays();
+                    wstep += 1;
+                    bool dead = false, wall = false;
+                    if (lane_in(actm)) {
+                        if (MULTI) {
+                            auto dim = [&]() {
+                                const DevLevel &L = llev[b.lev];
+                                return BulkDim{L.im, L.jm, L.km, (uint32_t)L.xoff, (uint32_t)L.poff};
+                            };
+                            dead = bulk_step<TM>(cm, sv, dim, xb, pb, b.dy, b.dz, tol, open, b, wall);
+                            if (!dead && wstep >= b.cap && b.kt != KT_WALL) {
+                                if (b.lev == cm.grid_num - 1) {
+                                    dead = true;
+                                } else {
+                                    /* coarsen the indices for the next grid level (:215-223) */
+                                    const DevLevel &L = llev[b.lev], &N = llev[b.lev + 1];
+                                    int ic, jc, kc;
+                                    bulk_cell(dim(), b, ic, jc, kc);
+                                    b.lev += 1;
+                                    bulk_place(dim(), coarsen(ic, L.cr[0], L.cmul[0]), coarsen(jc, L.cr[1], L.cmul[1]),
+                                               coarsen(kc, L.cr[2], L.cmul[2]), b);
+                                    b.dy = N.dy;
+                                    b.dz = N.dz;
+                                    bulk_load(xb, pb, b);
+                                    b.cap = wstep + bulk_cap(N.maxs);
+                                }
+                            }
+                        } else {
+                            auto dim = [&]() { return d0; };
+                            dead = bulk_step<TM>(cm, sv, dim, xb, pb, l0.dy, l0.dz, tol, open, b, wall);
+                            dead = dead || (wstep >= b.cap && b.kt != KT_WALL);
+                        }
+                    }
+                    const unsigned long long dm = __ballot(dead);
+                    bsteps += __popcll(actm & ~__ballot(wall));
+                    actm &= ~dm;
+                    pend |= dm;
                 }
             }
         }
@@ -689,23 +681,40 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
      * march; below that, the wavefront marches the remaining
      * rays one at a time, all lanes on one ray.  Then the
      * wavefront is done. */
-
-    if (active && wall) {
-        /* a ray still waiting at its wall: the wall's emission, and the ray is done */
-        const SnapView sv = snap_view(snaps + snap);
-        const DevLevel *lp = MULTI ? &llev[lev] : &snaps[snap].lev[0];
-        float Kw, Bw;
-        kb_pos<TM>(sv, e.row, e.rank, cm.nT, gld(lp->P, widx), Kw, Bw);
-        wall_hit(e, r, Bw, dacc);
-        finish_ray(cm, sl, seq, runit, rtid, rh, dacc, de);
-        nrays += 1;
-        active = false;
-        wall = 0;
-    }
-    if (__ballot(active) != 0ull) {
+    finish_pending();
+    bool active = lane_in(actm);
+    Ray r;
+    En e;
+    float dacc = b.dacc;
+    int lev = 0, counter = 0;
+    if (actm != 0ull) {
         const SnapView sv = snap_view(snaps + snap);
         DevLevel l0;
         if (!MULTI) l0 = level_view(&snaps[snap].lev[0]);
+        if (active) {
+            const DevLevel &L = MULTI ? llev[b.lev] : l0;
+            const BulkDim d{L.im, L.jm, L.km, MULTI ? (uint32_t)L.xoff : 0u, MULTI ? (uint32_t)L.poff : 0u};
+            e.row = b.rowb / (st * (TM == TAB_BF16 ? 4u : 8u));
+            e.rank = TM == TAB_BF16 ? (int)(b.rankb / (st * 16u)) : 0;
+            e.W = b.W; e.Bi = b.Bi; e.invBi = b.invBi;
+            r.xp = b.xp; r.yp = b.yp; r.zp = b.zp;
+            r.sx = b.sx; r.sy = b.sy; r.sz = b.sz;
+            r.isx = b.isx; r.isy = b.isy; r.isz = b.isz;
+            r.f0 = b.sx < 0.f; r.f1 = b.sy < 0.f; r.f2 = b.sz < 0.f;
+            r.tra = b.tra;
+            bulk_cell(d, b, r.ic, r.jc, r.kc);
+            lev = MULTI ? b.lev : 0;
+            counter = wstep - (b.cap - bulk_cap(L.maxs));
+            if (b.kt == KT_WALL) {
+                /* a ray still waiting at its wall: the wall's emission, and the ray is done */
+                float Kw, Bw;
+                kb_pos<TM>(sv, e.row, e.rank, cm.nT, ld_off<float>(MULTI ? sv.P_all : l0.P, b.cell4), Kw, Bw);
+                wall_hit(e, r, Bw, dacc);
+                finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), dacc, de);
+                active = false;
+            }
+        }
+        nrays += __popcll(actm);          /* every live ray ends here */
         /* the x faces of every level to LDS (the ray queue's
          * space, empty now), level g from xoff(g) */
         float *xul = reinterpret_cast<float *>(rq);
@@ -733,8 +742,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                     lev += 1;
                     counter = 0;
                 }
-                finish_ray(cm, sl, seq, runit, rtid, rh, dacc, de);
-                nrays += 1;
+                finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), dacc, de);
                 active = false;
             }
         } else {
@@ -746,8 +754,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                         march_ahead<TM, true>(cm, sv, l0, r, e, tol, dacc, counter, nsteps, xul,
                                               min(l0.maxs, counter + DRAIN_BLOCK));
                         if (!(r.tra > tol) || counter >= l0.maxs) {
-                            finish_ray(cm, sl, seq, runit, rtid, rh, dacc, de);
-                            nrays += 1;
+                            finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), dacc, de);
                             active = false;
                         }
                     }
@@ -760,9 +767,8 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                     int cc = bcast(counter, src), cs = 0;
                     march_coop<TM>(cm, sv, l0, cr, ce, tol, cd, cc, cs, xul, lane);
                     if (lane == src) {
-                        finish_ray(cm, sl, seq, runit, rtid, rh, cd, de);
+                        finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), cd, de);
                         nsteps += cs;
-                        nrays += 1;
                         active = false;
                     }
                 }
@@ -779,13 +785,10 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
     /* the drain's per-lane step counts stay 32-bit (a lane marches far
      * fewer than 2^32 steps: 1e13 steps over 16 k wavefronts is 1e7 per
      * lane); the wavefront's sums are 64-bit */
-    unsigned long long ws = (uint32_t)nsteps, wr = (uint32_t)nrays;
-    for (int o = 32; o > 0; o >>= 1) {
-        ws += __shfl_xor(ws, o);
-        wr += __shfl_xor(wr, o);
-    }
+    unsigned long long ws = (uint32_t)nsteps;
+    for (int o = 32; o > 0; o >>= 1) ws += __shfl_xor(ws, o);
     if (lane == 0) {
-        atomicAdd(&stats[0], wr);
+        atomicAdd(&stats[0], (unsigned long long)nrays);
         atomicAdd(&stats[1], ws + (unsigned long long)bsteps);
         atomicAdd(&stats[3], 64ull * (uint32_t)bsub);
         atomicAdd(&stats[4], (unsigned long long)bsteps);
@@ -877,8 +880,8 @@ static int default_wg_per_cu(const DevCommon &cm, int wg_per_cu) {
 }
 
 /* Defaults of the schedule (a refill mode < 0, a threshold or steps per
- * iteration <= 0).  Single grid: refills at 4 idle lanes, also between
- * the steps, 6 steps per iteration: within 1 % of the autotuner's pick at
+ * iteration <= 0).  Single grid: refills at 8 idle lanes (4: 2 % slower at
+ * 256x128x256), also between the steps, 6 steps per iteration: within 1 % of the autotuner's pick at
  * 256x128x256 (8 steps) and of the best at 64^3, where rays of 6 steps end
  * faster than the one round of 64 new rays per iteration replaces them at
  * 8 steps (0.60 of the lanes active, 10 % slower).
@@ -892,7 +895,7 @@ void batched_schedule(const DevCommon &cm, int &wg_per_cu, int &threshold, int &
     const bool mg = cm.grid_num > 1;
     if (refill < 0) refill = mg ? 0 : 1;
     wg_per_cu = default_wg_per_cu(cm, wg_per_cu);
-    if (threshold <= 0) threshold = 4;
+    if (threshold <= 0) threshold = mg ? 4 : 8;
     if (spi <= 0) spi = !mg ? (refill ? 6 : 3) : std::max(1, std::min(16, cm.maxs0));
 }
 

@@ -255,110 +255,6 @@ __device__ __forceinline__ void boundary(const DevCommon &cm, const S &sn, const
     }
 }
 
-/* The batched march carries the ray's linear cell index from step to step
- * (a step moves it by +-1, +-im or +-im jm) instead of forming it from the
- * three indices: the per-ray steps along y and z, set at the ray's start,
- * after a reflection or wrap and at a level change. */
-struct CellWalk {
-    uint32_t cell;
-    int dcy, dcz;
-};
-
-template <class G>
-__device__ __forceinline__ void cell_walk_setup(const G &L, const Ray &r, CellWalk &w) {
-    w.cell = (uint32_t)(r.ic - 1) + __umul24((uint32_t)L.im, (uint32_t)(r.jc - 1) +
-                                                              __umul24((uint32_t)L.jm, (uint32_t)(r.kc - 1)));
-    const int imjm = (int)__umul24((uint32_t)L.im, (uint32_t)L.jm);
-    w.dcy = r.f1 ? -L.im : L.im;
-    w.dcz = r.f2 ? -imjm : imjm;
-}
-
-/* The boundary condition of the batched march, without memory access:
- * periodic and specular faces move the ray on; at a black or bd 4 face the
- * ray keeps its transmissivity and gets the index of the wall's entry in
- * the level's position array (wall = 1), and the next march step takes the
- * wall's emission through the step's own table lookup (march_core_bulk);
- * a bd 5 face loses the ray (tra = 0, no tally).  The moves are those of
- * face_move, and they move the ray's cell walk with it; the wall entries
- * are wall_index's. */
-template <class G>
-__device__ __forceinline__ void boundary_defer(const DevCommon &cm, const G &L, Ray &r, bool left, int &wall,
-                                               uint32_t &widx, CellWalk &cw) {
-    /* one block per axis, each taken only when a lane left through one of
-     * its two faces; the face codes are wavefront-uniform */
-    const uint32_t im = (uint32_t)L.im, jm = (uint32_t)L.jm, km = (uint32_t)L.km;
-    const uint32_t imjm = __umul24(im, jm), ncell = __umul24(im, __umul24(jm, km));
-    const bool xo = left && (uint32_t)(r.ic - 1) >= im;
-    const bool yo = left && !xo && (uint32_t)(r.jc - 1) >= jm;
-    const bool zo = left && !xo && !yo;
-    if (xo) {
-        const bool lo = r.ic == 0;
-        const int bd = lo ? cm.bd[FW] : cm.bd[FE];
-        if (bd == 1) {                     /* periodic: to the opposite end */
-            r.ic = lo ? L.im : 1;
-            r.xp = lo ? cm.Lx : 0.f;
-            cw.cell += lo ? im : (uint32_t)-(int)im;
-        } else if (bd == 3) {              /* specular: back into the edge cell, sx reversed */
-            r.ic = lo ? 1 : L.im;
-            r.xp = lo ? 0.f : cm.Lx;
-            r.sx = -r.sx;
-            r.isx = -r.isx;
-            r.f0 = r.sx < 0.f;
-            cw.cell += lo ? 1u : (uint32_t)-1;
-        } else {                           /* black */
-            wall = 1;
-            widx = ncell + (lo ? 0u : __umul24(jm, km)) + (uint32_t)(r.jc - 1) +
-                   __umul24(jm, (uint32_t)(r.kc - 1));
-        }
-    }
-    if (yo) {
-        const bool lo = r.jc == 0;
-        const int bd = lo ? cm.bd[FS] : cm.bd[FN];
-        if (bd == 1) {
-            r.jc = lo ? L.jm : 1;
-            r.yp = lo ? cm.Ly : 0.f;
-            const uint32_t w = __umul24(jm, im);
-            cw.cell += lo ? w : (uint32_t)-(int)w;
-        } else if (bd == 3) {
-            r.jc = lo ? 1 : L.jm;
-            r.yp = lo ? 0.f : cm.Ly;
-            r.sy = -r.sy;
-            r.isy = -r.isy;
-            r.f1 = r.sy < 0.f;
-            cw.cell += lo ? im : (uint32_t)-(int)im;
-            cw.dcy = -cw.dcy;
-        } else {
-            wall = 1;
-            widx = ncell + 2u * __umul24(jm, km) + (lo ? 0u : __umul24(im, km)) +
-                   (uint32_t)(r.ic - 1) + __umul24(im, (uint32_t)(r.kc - 1));
-        }
-    }
-    if (zo) {
-        const bool lo = r.kc == 0;
-        const int bd = lo ? cm.bd[FB] : cm.bd[FT];
-        if (bd == 1) {
-            r.kc = lo ? L.km : 1;
-            r.zp = lo ? cm.Lz : 0.f;
-            const uint32_t w = ncell;
-            cw.cell += lo ? w : (uint32_t)-(int)w;
-        } else if (bd == 3) {
-            r.kc = lo ? 1 : L.km;
-            r.zp = lo ? 0.f : cm.Lz;
-            r.sz = -r.sz;
-            r.isz = -r.isz;
-            r.f2 = r.sz < 0.f;
-            cw.cell += lo ? imjm : (uint32_t)-(int)imjm;
-            cw.dcz = -cw.dcz;
-        } else if (bd == 2 || bd == 4) {
-            wall = 1;
-            widx = ncell + 2u * (__umul24(jm, km) + __umul24(im, km)) + (lo ? 0u : imjm) +
-                   (uint32_t)(r.ic - 1) + __umul24(im, (uint32_t)(r.jc - 1));
-        } else {                           /* bd 5: lost, no tally */
-            r.tra = 0.f;
-        }
-    }
-}
-
 /* The geometry of one march step (one iteration of march_ray's loop,
  * mc_gpu_noint.cu:252-654), given the x face the ray heads for
  * (fx = xu[ic - f0]): distances to the three candidate faces, the segment
@@ -457,73 +353,12 @@ __device__ __forceinline__ bool march_core(const DevCommon &cm, const S &sn, con
     return out;
 }
 
-/* A level of the batched march held per lane (the lanes of a multigrid
- * wavefront march rays on different levels): sizes, step cap, spacings and
- * the offsets of the level's x faces and table positions in the
- * snapshot's arrays of every level */
-struct LaneLevel {
-    int im, jm, km, maxs;
-    float dy, dz;
-    uint32_t xoff, poff;
-};
-
-__device__ __forceinline__ LaneLevel lane_level(const DevLevel &L) {
-    LaneLevel l;
-    l.im = L.im; l.jm = L.jm; l.km = L.km; l.maxs = L.maxs;
-    l.dy = L.dy; l.dz = L.dz;
-    l.xoff = (uint32_t)L.xoff; l.poff = (uint32_t)L.poff;
-    return l;
-}
-
 /* the index ic on the next level, (ic + r - 1) / r (mc_gpu_noint.cu:215-223),
  * by the level's multiplier */
 __device__ __forceinline__ int coarsen(int ic, int r, uint32_t m) {
     const uint32_t n = (uint32_t)(ic + r - 1);
     if (r == 1) return ic;
     return (int)(m ? __umulhi(n, m) : n / (uint32_t)r);
-}
-
-/* One step of the batched march.  A ray's table row is fixed, and along
- * its path the row t changes only every few cells, so the ray's last table
- * pair stays in registers and is loaded again only when t changes (kt: the
- * cached t, -1 for none; the loads of the other lanes are masked off).
- * The x face is loaded before the table position, so that the wait for the
- * position covers it and the geometry runs while a table pair is in
- * flight.  A ray waiting at a black wall (wall = 1, set by boundary_defer)
- * takes the wall's emission instead: the table at the wall's position,
- * with the whole transmissivity absorbed (optical depth infinite: alpha =
- * 1, the transmissivity then 0 and dumped), which is wall_hit's tally to
- * the bit; its geometry is discarded.  The cell index is carried in `cw`.
- * The level's x faces and positions are read at xu[xoff + i] and
- * P[poff + i], the indices clamped to xmax and pmax (a lane whose state is
- * stale reads in bounds).  Returns whether an index left the grid (never
- * for a wall step).  Same values as march_core and boundary, so the same
- * tallies. */
-template <int TM, class S, class G>
-__device__ __forceinline__ bool march_core_bulk(const DevCommon &cm, const S &sn, const G &L, const float *xu,
-                                                uint32_t xoff, uint32_t xmax, const float *P, uint32_t poff,
-                                                uint32_t pmax, Ray &r, const En &e, float tol, float &de, int &kt,
-                                                KbRaw &kc, bool wall, uint32_t widx, CellWalk &cw) {
-    const uint32_t ix = min(xoff + (uint32_t)(r.ic - r.f0), xmax);
-    const float fx = gld32(xu, ix);
-    asm volatile("" ::: "memory");
-    const float pos = gld32(P, min(poff + (wall ? widx : cw.cell), pmax));
-    int t;
-    ppos(pos, t, kc.a);
-    if (t != kt || wall) {
-        kb_load<TM>(sn, e.row, e.rank, cm.nT, t, kc);
-        kt = wall ? -1 : t;
-    }
-    const int stx = r.f0 ? -1 : 1;
-    float ds;
-    bool xa, ya;
-    const bool out = geo_move(L, r, fx, ds, xa, ya);
-    cw.cell += xa ? (uint32_t)stx : (uint32_t)(ya ? cw.dcy : cw.dcz);
-    float K, B;
-    kb_finish<TM>(kc, K, B);
-    int status = 0;
-    phys_core_x(wall ? -INFINITY : -(K * ds), B, e, tol, r.tra, de, status);
-    return out && !wall;
 }
 
 /* A ray marched on one grid level to its end, or until its step counter
