@@ -87,7 +87,8 @@ struct Unit {
     int s, n, v;          /* snapshot, cell (or wall cell) index, run     */
     int i, j, k, bound;   /* emission cell                               */
     uint32_t cid, tag;    /* Philox cell id and stream tag               */
-    float Ti;             /* emitting temperature                        */
+    int ti;               /* table row and weight of the emitting temperature */
+    float ai;
     int skip;             /* wall unit of a non-adiabatic wall           */
     uint32_t sh0, sh1;    /* Sobol sampler: the (cell, run)'s shift words */
 };
@@ -112,7 +113,7 @@ __device__ __forceinline__ Unit decode(const DevCommon &cm, const DevSnap *__res
         U.bound = 0;
         U.cid = (uint32_t)U.n + (uint32_t)sn.imax * sn.jmax * (sn.zstart - 1);
         U.tag = TAG_FLUID;
-        U.Ti = cell_T(sn, sn, U.i, U.j, U.k);
+        tpos(cell_T(sn, sn, U.i, U.j, U.k), sn.Tnb0, sn.invdT, cm.nT, U.ti, U.ai);
         if (cm.sampler) {
             const uint4 sh = draw4_bits(cm.k0, cm.k1, SOBOL_SHIFT_H, (uint32_t)U.v, U.cid, TAG_FLUID + 16u * (uint32_t)sn.snap);
             U.sh0 = sh.x;
@@ -127,7 +128,9 @@ __device__ __forceinline__ Unit decode(const DevCommon &cm, const DevSnap *__res
         U.cid = (uint32_t)m + (uint32_t)sn.jmax * (sn.zstart - 1);
         U.tag = U.bound ? TAG_EAST : TAG_WEST;
         U.skip = (U.bound == 0 && !cm.adiab[0]) || (U.bound == 1 && !cm.adiab[1]);
-        U.Ti = U.skip ? 0.f : wall_T(sn, sn, U.bound, U.j, U.k);
+        U.ti = 0;
+        U.ai = 0.f;
+        if (!U.skip) tpos(wall_T(sn, sn, U.bound, U.j, U.k), sn.Tnb0, sn.invdT, cm.nT, U.ti, U.ai);
     }
     return U;
 }
@@ -173,7 +176,7 @@ __device__ __forceinline__ Unit uni(const Unit &a) {
     Unit b;
     b.s = uni(a.s); b.n = uni(a.n); b.v = uni(a.v);
     b.i = uni(a.i); b.j = uni(a.j); b.k = uni(a.k); b.bound = uni(a.bound);
-    b.cid = uni(a.cid); b.tag = uni(a.tag); b.Ti = uni(a.Ti); b.skip = uni(a.skip);
+    b.cid = uni(a.cid); b.tag = uni(a.tag); b.ti = uni(a.ti); b.ai = uni(a.ai); b.skip = uni(a.skip);
     b.sh0 = uni(a.sh0); b.sh1 = uni(a.sh1);
     return b;
 }
@@ -213,9 +216,10 @@ struct SlotTally {
     int done, tid;
 };
 struct SlotPlace {
-    int ic, jc, kc;
     float xp, yp, zp;
-    int pad0, pad1;
+    uint32_t cell4, ix4;      /* byte offsets of the cell and of its high x face */
+    float jc, kc;
+    int ic;
 };
 struct Slots {
     SlotTally *tal;
@@ -244,7 +248,7 @@ __device__ __forceinline__ void q_put(uint32_t *q, int qs, float sx, float sy, f
 template <bool SURF, int TM>
 __device__ __forceinline__ void q_get(const uint32_t *q, int qs, const Slots &sl, const DevSnap &sn, const BulkDim &dim,
                                       uint32_t st, int wstep, int maxs, BulkRay &b) {
-    const uint4 *rec = reinterpret_cast<const uint4 *>(q + qs * QREC);
+    const uint4 *rec = reinterpret_cast<const uint4 *>(q + __umul24((uint32_t)qs, (uint32_t)QREC));
     const uint4 ra = rec[0], rb = rec[1], rc = rec[2];
     b.sx = __uint_as_float(ra.x);
     b.sy = __uint_as_float(ra.y);
@@ -262,19 +266,22 @@ __device__ __forceinline__ void q_get(const uint32_t *q, int qs, const Slots &sl
     b.tid = (int)rc.w;
     const uint4 *pr = reinterpret_cast<const uint4 *>(&sl.pl[rc.z & (NSLOT - 1)]);
     const uint4 p0 = pr[0], p1 = pr[1];
-    Ray r;
-    r.ic = (int)p0.x; r.jc = (int)p0.y; r.kc = (int)p0.z;
-    r.xp = __uint_as_float(p0.w); r.yp = __uint_as_float(p1.x); r.zp = __uint_as_float(p1.y);
-    if (SURF) {
-        r.f0 = b.sx < 0.f; r.f1 = b.sy < 0.f; r.f2 = b.sz < 0.f;
-        surface_adjust(sn, r);
-    }
-    b.xp = r.xp; b.yp = r.yp; b.zp = r.zp;
+    b.xp = __uint_as_float(p0.x); b.yp = __uint_as_float(p0.y); b.zp = __uint_as_float(p0.z);
     b.tra = 1.0f;
     b.dacc = 0.f;
     b.kt = KT_NONE;
     b.cap = wstep + bulk_cap(maxs);
-    bulk_place(dim, r.ic, r.jc, r.kc, b);
+    if (SURF) {
+        Ray r;
+        r.ic = (int)p1.w; r.jc = (int)__uint_as_float(p1.y); r.kc = (int)__uint_as_float(p1.z);
+        r.xp = b.xp; r.yp = b.yp; r.zp = b.zp;
+        r.f0 = b.sx < 0.f; r.f1 = b.sy < 0.f; r.f2 = b.sz < 0.f;
+        surface_adjust(sn, r);
+        bulk_place(dim, r.ic, r.jc, r.kc, b);
+    } else {
+        b.cell4 = p0.w;
+        bulk_heads(dim, p1.x, __uint_as_float(p1.y), __uint_as_float(p1.z), b);
+    }
 }
 
 /* the distance from unit number u (16 bits, as the ray records hold it)
@@ -493,8 +500,8 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                         }
                         __syncthreads();
                         radix_offsets(hist, lane);
-                        radix_pass(kr, ka, hist, P, 0, lane);
-                        radix_pass(ka, kr, hist + 256, P, 8, lane);
+                        radix_first(kr, ka, hist, P, lane);
+                        radix_high(ka, kr, hist + 256, P, radix_high_bits(cm.nB * cm.nQ), lane);
                     }
                 }
             }
@@ -529,9 +536,14 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                     t.done = 0;
                     t.tid = tidx;
                     SlotPlace &pl = sl.pl[cslot];
+                    const DevLevel &L = sn.lev[0];
                     pl.ic = SURF ? (U.bound ? sn.imax : 1) : U.i;
-                    pl.jc = U.j;
-                    pl.kc = U.k;
+                    pl.jc = (float)U.j;
+                    pl.kc = (float)U.k;
+                    pl.ix4 = 4u * (uint32_t)((MULTI ? L.xoff : 0) + pl.ic);
+                    pl.cell4 = 4u * ((MULTI ? (uint32_t)L.poff : 0u) + (uint32_t)(pl.ic - 1) +
+                                     __umul24((uint32_t)L.im, (uint32_t)(U.j - 1) +
+                                                                  __umul24((uint32_t)L.jm, (uint32_t)(U.k - 1))));
                     pl.xp = SURF ? (U.bound ? cm.Lx : 0.f) : gld(sn.x0, U.i);
                     pl.yp = gld(sn.y0, U.j);
                     pl.zp = gld(sn.z0, U.k);
@@ -578,7 +590,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                     if (SURF) surface_dir(a, b, U.bound, sx, sy, sz);
                     else fluid_dir(a, b, sx, sy, sz);
                     En ge;
-                    energy<TM>(cm, sn, key, U.Ti, SURF, U.bound, ge);
+                    energy_ta<TM>(cm, sn, key, U.ti, U.ai, SURF, U.bound, ge);
                     q_put(rq, qwrap(qhead + qcount + lane), sx, sy, sz, ge, key, cunit, ctid, h);
                 }
                 __syncthreads();

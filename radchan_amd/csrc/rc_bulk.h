@@ -76,19 +76,26 @@ struct BulkRay {
 /* steps to the cap of a level, bounded so that the count cannot overflow */
 __device__ __forceinline__ int bulk_cap(int maxs) { return min(maxs, 1 << 30); }
 
-/* the ray's place on a level: cell (ic, jc, kc), direction signs from s */
-__device__ __forceinline__ void bulk_place(const BulkDim &d, int ic, int jc, int kc, BulkRay &b) {
+/* what the direction's signs decide at the cell with high x face ix4 and
+ * indices (jc, kc): the faces ahead, where the ray leaves the grid, and the
+ * cell's steps */
+__device__ __forceinline__ void bulk_heads(const BulkDim &d, uint32_t ix4, float jc, float kc, BulkRay &b) {
     const bool nx = b.sx < 0.f, ny = b.sy < 0.f, nz = b.sz < 0.f;
     const int imjm4 = 4 * (int)__umul24((uint32_t)d.im, (uint32_t)d.jm);
     b.dx4 = nx ? -4 : 4;
-    b.ix4 = 4u * (d.xoff + (uint32_t)(ic - (nx ? 1 : 0)));
-    b.xlim = 4u * (d.xoff + (nx ? 0xFFFFFFFFu : (uint32_t)(d.im + 1)));
-    b.jf = (float)(jc - (ny ? 1 : 0));
-    b.kf = (float)(kc - (nz ? 1 : 0));
+    b.ix4 = nx ? ix4 - 4u : ix4;
+    b.xlim = nx ? 4u * d.xoff - 4u : 4u * (d.xoff + (uint32_t)(d.im + 1));
+    b.jf = jc + (ny ? -1.0f : 0.0f);
+    b.kf = kc + (nz ? -1.0f : 0.0f);
     b.jlim = ny ? -1.0f : (float)(d.jm + 1);
     b.klim = nz ? -1.0f : (float)(d.km + 1);
     b.dcy4 = ny ? -4 * d.im : 4 * d.im;
     b.dcz4 = nz ? -imjm4 : imjm4;
+}
+
+/* the ray's place on a level: cell (ic, jc, kc), direction signs from s */
+__device__ __forceinline__ void bulk_place(const BulkDim &d, int ic, int jc, int kc, BulkRay &b) {
+    bulk_heads(d, 4u * (d.xoff + (uint32_t)ic), (float)jc, (float)kc, b);
     b.cell4 = 4u * (d.poff + (uint32_t)(ic - 1) +
                     __umul24((uint32_t)d.im, (uint32_t)(jc - 1) + __umul24((uint32_t)d.jm, (uint32_t)(kc - 1))));
 }

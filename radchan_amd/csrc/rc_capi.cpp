@@ -34,7 +34,7 @@ using namespace rc;
 
 namespace {
 
-constexpr int kGuideM = 2048;   /* guide-table resolution for the band CDFs */
+constexpr int kGuideM = 2048;   /* guide-table resolution for the band CDFs (a power of two) */
 
 /* a roctx range over the enclosing scope (set-up, launch and harvest
  * phases show up on a rocprofv3 --marker-trace timeline; no cost without
@@ -107,7 +107,9 @@ struct SnapState {
     float Tmax = 0.f, kappamax = 0.f, Ibmax = 0.f, Ibmax_w = 0.f, Ibmax_e = 0.f;
     double kappamax64 = 0.0, Ibmax64 = 0.0, Ibmax_w64 = 0.0, Ibmax_e64 = 0.0;   /* the FP64 path's */
     int tm = 0, tstar = 0;
-    DevBuf T0, cdf_b, cdf_g, cdf_bs, guide_b, guide_bs;
+    DevBuf T0, cdf_b, cdf_g, cdf_g4, cdf_bs, guide_b, guide_bs;
+    bool g4 = false;                      /* cdf_g4 holds the g CDFs' quarters */
+    DevBuf kbm;                           /* k and Ib of every table row at Tmax */
     DevBuf Pall;                          /* table positions of every level (DevLevel.P) */
     DevBuf Tall;                          /* FP64 path: the temperatures behind Pall */
     std::unique_ptr<TableSet> grey;     /* grey runs: tables follow Tmax */
@@ -386,6 +388,14 @@ int snapshot_rows(rc_ctx *c, const Tables &t, SnapState &s) {
         }
         return g;
     };
+    /* the g CDFs' quarters (launch_rows_derived) serve where a two-level
+     * search finds what the count over the row does: 16 entries,
+     * non-decreasing */
+    s.g4 = nQ == 16;
+    for (size_t i = 0; s.g4 && i < cg.size(); ++i) s.g4 = i % 16 == 0 ? cg[i] == cg[i] : cg[i] >= cg[i - 1];
+    if (s.g4)
+        if (int e = s.cdf_g4.ensure((size_t)nB * 16)) return e;
+    if (int e = s.kbm.ensure((size_t)nB * nQ * 8)) return e;
     if (int e = upload(s.guide_b, guide(cb), c->stream)) return e;
     if (int e = upload(s.guide_bs, guide(cs), c->stream)) return e;
     if (int e = upload(s.cdf_b, cb, c->stream)) return e;
@@ -400,6 +410,7 @@ DevCommon make_common(const rc_ctx *c) {
     cm.imax = p.imax; cm.jmax = p.jmax; cm.kmax = p.kmax; cm.kloc = c->kloc; cm.zstart = c->zstart;
     cm.nVar = p.nVar; cm.photmax = p.photmax; cm.srt = (p.srt == 1 && !p.grey) ? 1 : 0;
     cm.nB = p.nB; cm.nQ = p.nQ; cm.nT = p.nT; cm.grid_num = p.grid_num;
+    cm.qmul = p.nQ > 1 ? (uint32_t)((((uint64_t)1 << 32) + (uint64_t)p.nQ - 1) / (uint64_t)p.nQ) : 0u;
     cm.ncell = c->ncell; cm.nsurf = c->nsurf;
     cm.Lx = p.Lx; cm.Ly = p.Ly; cm.Lz = p.Lz; cm.toll = p.toll; cm.tollS = p.tollS;
     for (int f = 0; f < 6; ++f) cm.bd[f] = p.bd[f];
@@ -427,6 +438,8 @@ int push_snaps(rc_ctx *c) {
         d.kp16 = ts.kp16.as<uint32_t>(); d.bp = ts.bp.as<float4>();
         d.cdf_b = S.cdf_b.as<float>(); d.cdf_g = S.cdf_g.as<float>(); d.cdf_bs = S.cdf_bs.as<float>();
         d.cdf_gs = ts.cdf_gs.as<float>(); d.rank_of = ts.rank_of.as<int>();
+        d.cdf_g4 = S.g4 ? S.cdf_g4.as<float4>() : nullptr;
+        d.kbm = S.kbm.as<float2>();
         d.guide_b = S.guide_b.as<int>(); d.guide_bs = S.guide_bs.as<int>(); d.gM = kGuideM;
         d.T0 = S.T0.as<float>();
         d.xu_all = c->xuall.as<float>();
@@ -471,7 +484,10 @@ int push_snaps(rc_ctx *c) {
         v[s] = d;
     }
     c->hsnap = v;
-    return upload(c->dsnap, c->hsnap, c->stream);
+    if (int e = upload(c->dsnap, c->hsnap, c->stream)) return e;
+    launch_rows_derived(c->stream, make_common(c), c->dsnap.as<DevSnap>(), (int)v.size());
+    RC_HIP(hipGetLastError());
+    return 0;
 }
 
 }  // namespace

@@ -230,13 +230,13 @@ __device__ __forceinline__ int upper_bound(const float *__restrict__ cdf, int n,
 }
 
 /* upper_bound with a guide table g[m] = first index with cdf > m/M
- * (Chen and Asau, 1974): the answer lies in [g[m-1], g[m+2]] for
- * m = floor(R M), one slot of slack either side against rounding of R M.
- * Returns exactly what upper_bound returns. */
+ * (Chen and Asau, 1974), M a power of two: R M is exact, so the answer lies
+ * in [g[m], g[m+1]] for m = floor(R M).  Returns exactly what upper_bound
+ * returns. */
 __device__ __forceinline__ int upper_bound_guided(const float *__restrict__ cdf, int n, const int *__restrict__ g,
                                                   int M, float R) {
     int m = (int)(R * (float)M);
-    int lo = gld(g, max(m - 1, 0)), hi = gld(g, min(m + 2, M));
+    int lo = gld(g, m), hi = gld(g, min(m + 1, M));
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
         if (R < gld(cdf, mid)) hi = mid; else lo = mid + 1;
@@ -263,6 +263,17 @@ __device__ __forceinline__ int upper_bound_short(const float *__restrict__ cdf, 
     if (R == 1.0f) c = n - 1;
     if (c > n - 1) c = n - 1;
     return c;
+}
+
+/* upper_bound_short of a non-decreasing row of 16 entries, c its entries 3,
+ * 7 and 11: the quarter first, then its four entries (7 comparisons and 32
+ * bytes instead of 16 and 64) */
+__device__ __forceinline__ int upper_bound_16(const float *__restrict__ cdf, float4 c, float R) {
+    const int q = ((c.x <= R) ? 1 : 0) + ((c.y <= R) ? 1 : 0) + ((c.z <= R) ? 1 : 0);
+    const float4 v = gld(reinterpret_cast<const float4 *>(cdf), q);
+    int n = 4 * q + ((v.x <= R) ? 1 : 0) + ((v.y <= R) ? 1 : 0) + ((v.z <= R) ? 1 : 0) + ((v.w <= R) ? 1 : 0);
+    if (R == 1.0f) n = 15;
+    return min(n, 15);
 }
 
 __device__ __forceinline__ float lerp(float a, float b, float w) { return fmaf(w, b - a, a); }

@@ -20,6 +20,7 @@ enum { TAG_FLUID = 0, TAG_WEST = 1, TAG_EAST = 2, TAG_NOISE = 3 };
 struct DevCommon {
     int imax, jmax, kmax, kloc, zstart;
     int nVar, photmax, srt, nB, nQ, nT, grid_num;
+    uint32_t qmul;                 /* key / nQ = umulhi(key, qmul) for keys below 2^16; 0: nQ = 1 */
     int ncell, nsurf;              /* emitting fluid cells, wall cells per wall */
     float Lx, Ly, Lz, toll, tollS;
     int bd[6], adiab[2];
@@ -90,7 +91,10 @@ struct DevSnap {
     const float *cdf_g;            /* [nB][nQ] g CDFs, row t*             */
     const float *cdf_bs;           /* [nB] wall band CDF, row t*          */
     const float *cdf_gs;           /* [nQ] cumulative quadrature weights  */
+    const float4 *cdf_g4;          /* [nB] entries 3, 7, 11 of the g CDF (nQ = 16, every row */
+                                   /* non-decreasing; else nullptr)       */
     const int *rank_of;            /* [nB] sorted rank of each band       */
+    const float2 *kbm;             /* [nB nQ] k and Ib of each row at Tmax */
     const int *guide_b;            /* [gM+1] first index with cdf_b > m/gM */
     const int *guide_bs;           /* [gM+1] same for cdf_bs               */
     int gM, pad2;
@@ -159,6 +163,9 @@ void batched_schedule(const DevCommon &cm, int &wg_per_cu, int &threshold, int &
 size_t batched_srt_keys(const DevCommon &cm, long nunit_cells, int wg_per_cu);
 void launch_zero(hipStream_t st, double *p, size_t n);
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n);
+/* k and Ib of every table row at each snapshot's Tmax, to its kbm, and the
+ * quarter entries of its g CDFs, to its cdf_g4 */
+void launch_rows_derived(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int nsnap);
 /* input check and Tmax of a temperature field on the device (out: 2 words) */
 void launch_field_scan(hipStream_t st, const float *T, int imax, int jmax, int kmax, uint32_t *out);
 

@@ -26,9 +26,16 @@ using namespace rcd;
 __device__ __forceinline__ uint32_t band_key(const DevCommon &cm, const DevSnap &sn, bool surface, float u2, float u3) {
     const int nb = surface ? upper_bound_guided(sn.cdf_bs, cm.nB, sn.guide_bs, sn.gM, u2)
                            : upper_bound_guided(sn.cdf_b, cm.nB, sn.guide_b, sn.gM, u2);
+    const uint32_t row = __umul24((uint32_t)gld(sn.rank_of, nb), (uint32_t)cm.nQ);
+    if (!surface && sn.cdf_g4) return row + (uint32_t)upper_bound_16(sn.cdf_g + 16 * (size_t)nb, gld(sn.cdf_g4, nb), u3);
     const float *gc = surface ? sn.cdf_gs : sn.cdf_g + (size_t)nb * cm.nQ;
     const int g = (cm.nQ <= 32) ? upper_bound_short(gc, cm.nQ, u3) : upper_bound(gc, cm.nQ, u3);
-    return (uint32_t)(gld(sn.rank_of, nb) * cm.nQ + g);
+    return row + (uint32_t)g;
+}
+
+/* the sorted band rank of a key, key / nQ */
+__device__ __forceinline__ int key_rank(const DevCommon &cm, uint32_t key) {
+    return (int)(cm.qmul ? __umulhi(key, cm.qmul) : key);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -677,20 +684,31 @@ __device__ __forceinline__ void march_all(const DevCommon &cm, const DevSnap &sn
 }
 
 /* per-ray energy constants: W = Ibmax B(Ti)/B(Tmax) K(Ti)/K(Tmax) for the
- * fluid (:181-186), W = Ibmax_s B(Tw)/B(Tmax) for walls (:1419-1424) */
+ * fluid (:181-186), W = Ibmax_s B(Tw)/B(Tmax) for walls (:1419-1424); the
+ * emitting temperature as its table row ti and weight ai, the values at
+ * Tmax from the snapshot's row table (neighbouring keys, one cache line) */
+template <int TM = TAB_RT>
+__device__ __forceinline__ void energy_ta(const DevCommon &cm, const DevSnap &sn, uint32_t key, int ti, float ai,
+                                          bool surface, int bound, En &e) {
+    e.rank = key_rank(cm, key);
+    e.row = key;
+    float Ki, Bi;
+    kb_ta<TM>(sn, e.row, e.rank, cm.nT, ti, ai, Ki, Bi);
+    const float2 m = gld32(sn.kbm, key);
+    e.Bi = Bi;
+    e.invBi = 1.0f / Bi;
+    if (!surface) e.W = sn.Ibmax * (((Bi / m.y) * Ki) / m.x);
+    else e.W = (bound ? sn.Ibmax_e : sn.Ibmax_w) * (Bi / m.y);
+}
+
+/* the same at temperature Ti */
 template <int TM = TAB_RT>
 __device__ __forceinline__ void energy(const DevCommon &cm, const DevSnap &sn, uint32_t key, float Ti, bool surface,
                                        int bound, En &e) {
-    const int rank = (int)(key / (uint32_t)cm.nQ);
-    e.rank = rank;
-    e.row = key;
-    float Ki, Bi, Km, Bm;
-    kb_at<TM>(sn, e.row, rank, cm.nT, Ti, Ki, Bi);
-    kb_at<TM>(sn, e.row, rank, cm.nT, sn.Tmax, Km, Bm);
-    e.Bi = Bi;
-    e.invBi = 1.0f / Bi;
-    if (!surface) e.W = sn.Ibmax * (((Bi / Bm) * Ki) / Km);
-    else e.W = (bound ? sn.Ibmax_e : sn.Ibmax_w) * (Bi / Bm);
+    int ti;
+    float ai;
+    tpos(Ti, sn.Tnb0, sn.invdT, cm.nT, ti, ai);
+    energy_ta<TM>(cm, sn, key, ti, ai, surface, bound, e);
 }
 
 /* emitting fluid cell n -> (i, j, k global) */

@@ -178,6 +178,23 @@ __global__ void __launch_bounds__(256) k_pos_from_T(const float *__restrict__ Tl
     }
 }
 
+/* k and Ib of every table row at the snapshot's Tmax (the rays' emission
+ * weights divide by them): one pass per field instead of one gather, a
+ * table position and two interpolations per ray; and entries 3, 7 and 11 of
+ * every g CDF of 16 */
+__global__ void __launch_bounds__(256) k_rows_derived(DevCommon cm, const DevSnap *__restrict__ snaps) {
+    const DevSnap &sn = snaps[blockIdx.y];
+    const int row = blockIdx.x * blockDim.x + threadIdx.x;
+    if (row >= cm.nB * cm.nQ) return;
+    float K, B;
+    kb_at(sn, (uint32_t)row, key_rank(cm, (uint32_t)row), cm.nT, sn.Tmax, K, B);
+    const_cast<float2 *>(sn.kbm)[row] = make_float2(K, B);
+    if (sn.cdf_g4 && row < cm.nB) {
+        const float *g = sn.cdf_g + 16 * (size_t)row;
+        const_cast<float4 *>(sn.cdf_g4)[row] = make_float4(g[3], g[7], g[11], 0.f);
+    }
+}
+
 /* ------------------------------------------------------------------------ */
 /* the srt enumeration                                                       */
 
@@ -239,8 +256,8 @@ __global__ void __launch_bounds__(64) k_sort_bands(DevCommon cm, const DevSnap *
             }
             __syncthreads();
             radix_offsets(hist, lane);
-            radix_pass(ka, kb, hist, P, 0, lane);
-            radix_pass(kb, ka, hist + 256, P, 8, lane);
+            radix_first(ka, kb, hist, P, lane);
+            radix_high(kb, ka, hist + 256, P, radix_high_bits(cm.nB * cm.nQ), lane);
             for (int h = lane; h < P; h += 64) keys[(size_t)u * P + h] = ka[h];
             __syncthreads();
         }
@@ -522,6 +539,10 @@ void launch_pos_from_T(hipStream_t st, const rc_params &p, int g, const float *T
     const int blocks = (int)std::min<size_t>((n + 255) / 256, 65536);
     hipLaunchKernelGGL(k_pos_from_T, dim3(blocks), dim3(256), 0, st, Tl, Tw, p.maxi[g], p.maxj[g], p.maxk[g],
                        face_modes(p), Tnb0, invdT, nT, P, Tout);
+}
+
+void launch_rows_derived(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int nsnap) {
+    hipLaunchKernelGGL(k_rows_derived, dim3((cm.nB * cm.nQ + 255) / 256, nsnap), dim3(256), 0, st, cm, snaps);
 }
 
 void launch_sort(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v, int surface, int nunit,
