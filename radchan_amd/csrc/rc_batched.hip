@@ -181,9 +181,6 @@ __device__ __forceinline__ Unit uni(const Unit &a) {
     return b;
 }
 
-/* device unit queue: counters of the QPARTS ranges (fluid at queue[0..],
- * walls at queue[16..]) */
-constexpr int QPARTS = 8;
 constexpr int QRAYS = 800;       /* rays per request to the queue, but one chunk at least */
 
 /* LDS ray queue: rays generated in bulk (all 64 lanes) wait here until an
@@ -426,22 +423,28 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
              * chunks are split into QPARTS contiguous ranges (z slabs of
              * the field), one per XCD, each with its own counter, so that
              * an XCD's L2 holds its own slab; a range that runs out sends
-             * the wavefront to the next one.  One counter serves about 11
-             * requests per microsecond, whoever asks, so a request takes
-             * several chunks while the range holds plenty: half of its
+             * the wavefront to the next one.  A counter serves a
+             * limited number of requests per microsecond, whoever asks
+             * (QSTRIDE), so a request takes several chunks while the range holds plenty: half of its
              * even share of what was left at its last request (guided
              * self-scheduling), between 1 and as many as hold QRAYS rays
              * (at most 16).  192x128x192 and 100 rays per unit, three
-             * levels: with one chunk per request the counters alone took
-             * 54 ms, for one or two runs per cell alike; now 23.7 and
-             * 47.1 ms.  QRAYS: 400 to 1600 are within 1 % of each other;
+             * levels: with one chunk per request (and the counters in one
+             * cache line) they alone took 54 ms, for one or two runs per
+             * cell alike; now 23.7 and 47.1 ms.  QRAYS: 400 to 1600 are within 1 % of each other;
              * without the bound in rays, units of 6000 rays ended 17 %
              * later (28x96x128, the last wavefronts' chunks). */
             while (cleft == 0 && part >= 0) {
                 const int pb = (int)((long)nch * part / QPARTS), pe = (int)((long)nch * (part + 1) / QPARTS);
                 const int ask = min(max((pe - pb - plast) / (2 * pwaves), 1), askmax);
+                /* a range other than the wavefront's own is looked at before
+                 * it is asked: near the end every wavefront passes by every
+                 * counter, and loads of one line do not queue up */
                 int c0 = 0;
-                if (lane == 0) c0 = atomicAdd(&queue[part], ask);
+                if (lane == 0) {
+                    if (ptries) c0 = __hip_atomic_load(&queue[part * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (pb + c0 < pe) c0 = atomicAdd(&queue[part * QSTRIDE], ask);
+                }
                 c0 = uni(c0);
                 if (pb + c0 < pe) {
                     plast = c0 + ask;
@@ -815,11 +818,11 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
      * lane); the wavefront's sums are 64-bit */
     unsigned long long ws = (uint32_t)nsteps;
     for (int o = 32; o > 0; o >>= 1) ws += __shfl_xor(ws, o);
-    if (lane == 0) {
-        atomicAdd(&stats[0], (unsigned long long)nrays);
-        atomicAdd(&stats[1], ws + (unsigned long long)bsteps);
-        atomicAdd(&stats[3], 64ull * (uint32_t)bsub);
-        atomicAdd(&stats[4], (unsigned long long)bsteps);
+    if (lane == 0 && nrays) {
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)nrays);
+        atomicAdd(&stat_line(stats)[1], ws + (unsigned long long)bsteps);
+        atomicAdd(&stat_line(stats)[3], 64ull * (uint32_t)bsub);
+        atomicAdd(&stat_line(stats)[4], (unsigned long long)bsteps);
     }
 }
 
@@ -954,7 +957,7 @@ void launch_batched(hipStream_t st, const DevCommon &cm0, const DevSnap *snaps, 
     const size_t lds = (size_t)batched_lds_words(n2, cm.srt, cm.grid_num > 1) * 4;
     const size_t nde = (size_t)nunit_cells * cm.nVar;
     const int grid = batched_grid(cm, nunit_cells, wg_per_cu);
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, queue, QPARTS);
+    hipLaunchKernelGGL(k_zero_int, dim3(2), dim3(256), 0, st, queue, QUEUE_WORDS);
     launch_zero(st, de, nde);
     const bool multi = cm.grid_num > 1;
     const bool bf = snaps_bf16;

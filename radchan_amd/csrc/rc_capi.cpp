@@ -673,7 +673,7 @@ rc_ctx *rc_create(const rc_params *pp) {
     if (upload(c->x0, c->grids[0].x, c->stream) || upload(c->y0, c->grids[0].y, c->stream) ||
         upload(c->z0, c->grids[0].z, c->stream))
         return nullptr;
-    if (c->stats.ensure(8 * sizeof(unsigned long long)) || c->queue.ensure(64 * sizeof(int))) return nullptr;
+    if (c->stats.ensure(STAT_WORDS * sizeof(unsigned long long)) || c->queue.ensure(2 * QUEUE_WORDS * sizeof(int))) return nullptr;
     if (hipStreamSynchronize(c->stream) != hipSuccess) { set_error("stream synchronize failed"); return nullptr; }
     return c.release();
 }
@@ -800,7 +800,7 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
     const DevSnap *ds = c->dsnap.as<DevSnap>();
     const bool walls = p.calcwalls == 1 && (p.adiabw == 1 || p.adiabe == 1);
     int n = 0;
-    launch_zero_u64(c->stream, c->stats.as<unsigned long long>(), 8);
+    launch_zero_u64(c->stream, c->stats.as<unsigned long long>(), STAT_WORDS);
     ++n;
     if (timed) RC_HIP(hipEventRecord(c->evm0, c->stream));
     if (variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) {
@@ -852,7 +852,7 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
         }
         if (walls) {
             launch_batched(c->stream, cw, ds, nsnap, nsnap * 2 * c->nsurf, 1, c->table_bf16, c->ds.as<double>(),
-                           c->stats.as<unsigned long long>(), c->queue.as<int>() + 16, c->wg_per_cu, c->threshold,
+                           c->stats.as<unsigned long long>(), c->queue.as<int>() + QUEUE_WORDS, c->wg_per_cu, c->threshold,
                            c->spi);
             n += 3;
             if (c->reduction == 1) {
@@ -1105,6 +1105,18 @@ int rc_autotune(rc_ctx *c, int32_t *best_wg, int32_t *best_th, int32_t *best_spi
     return 0;
 }
 
+/* the counters' copies (STAT_LINES) summed into the statistics */
+static int read_stats(const DevBuf &stats, rc_stats &out) {
+    unsigned long long h[STAT_WORDS];
+    RC_HIP(hipMemcpy(h, stats.p, sizeof h, hipMemcpyDeviceToHost));
+    int64_t *const to[5] = {&out.rays, &out.steps, &out.capped, &out.bulk_slots, &out.bulk_steps};
+    for (int i = 0; i < 5; ++i) {
+        *to[i] = 0;
+        for (int l = 0; l < STAT_LINES; ++l) *to[i] += (int64_t)h[l * STAT_STRIDE + i];
+    }
+    return 0;
+}
+
 int rc_sync(rc_ctx *c, rc_stats *st) {
     const Range range_("radchan: harvest (rc_sync)");
     if (!c) { set_error("null context"); return -1; }
@@ -1113,15 +1125,9 @@ int rc_sync(rc_ctx *c, rc_stats *st) {
         float ms = 0.f, mms = 0.f;
         RC_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
         RC_HIP(hipEventElapsedTime(&mms, c->evm0, c->evm1));
-        unsigned long long h[8];
-        RC_HIP(hipMemcpy(h, c->stats.p, sizeof h, hipMemcpyDeviceToHost));
+        if (int e = read_stats(c->stats, c->last)) return e;
         c->last.kernel_ms = ms;
         c->last.march_ms = mms;
-        c->last.rays = (int64_t)h[0];
-        c->last.steps = (int64_t)h[1];
-        c->last.capped = (int64_t)h[2];
-        c->last.bulk_slots = (int64_t)h[3];
-        c->last.bulk_steps = (int64_t)h[4];
         c->launched = false;
     }
     if (st) *st = c->last;
@@ -1360,8 +1366,8 @@ int rc_group_run(rc_group *g) {
     if (int e = upload(g->dsnap, g->h, g->stream)) return e;
     if (int e = g->de.ensure((size_t)cells * nVar * 8)) return e;
     if (walls) { if (int e = g->ds.ensure((size_t)wcells * nVar * 8)) return e; }
-    if (int e = g->stats.ensure(8 * sizeof(unsigned long long))) return e;
-    if (int e = g->queue.ensure(32 * sizeof(int))) return e;
+    if (int e = g->stats.ensure(STAT_WORDS * sizeof(unsigned long long))) return e;
+    if (int e = g->queue.ensure(2 * QUEUE_WORDS * sizeof(int))) return e;
     DevCommon cm = make_common(c0);
     cm.refill = g->refill;
     const size_t nk = std::max(batched_srt_keys(cm, cells, g->wg_per_cu),
@@ -1371,7 +1377,7 @@ int rc_group_run(rc_group *g) {
     cm.srt_keys = g->srtk.as<uint16_t>();
     int n = 0;
     RC_HIP(hipEventRecord(g->ev0, g->stream));
-    launch_zero_u64(g->stream, g->stats.as<unsigned long long>(), 8);
+    launch_zero_u64(g->stream, g->stats.as<unsigned long long>(), STAT_WORDS);
     ++n;
     RC_HIP(hipEventRecord(g->evm0, g->stream));
     launch_batched(g->stream, cm, g->dsnap.as<DevSnap>(), (int)g->h.size(), cells, 0, c0->table_bf16,
@@ -1380,7 +1386,7 @@ int rc_group_run(rc_group *g) {
     n += 3;
     if (walls) {
         launch_batched(g->stream, cm, g->dsnap.as<DevSnap>(), (int)g->h.size(), wcells, 1, c0->table_bf16,
-                       g->ds.as<double>(), g->stats.as<unsigned long long>(), g->queue.as<int>() + 16,
+                       g->ds.as<double>(), g->stats.as<unsigned long long>(), g->queue.as<int>() + QUEUE_WORDS,
                        g->wg_per_cu, g->threshold, g->spi);
         n += 3;
     }
@@ -1423,15 +1429,9 @@ int rc_group_sync(rc_group *g, rc_stats *st) {
         float ms = 0.f, mms = 0.f;
         RC_HIP(hipEventElapsedTime(&ms, g->ev0, g->ev1));
         RC_HIP(hipEventElapsedTime(&mms, g->evm0, g->evm1));
-        unsigned long long h[8];
-        RC_HIP(hipMemcpy(h, g->stats.p, sizeof h, hipMemcpyDeviceToHost));
+        if (int e = read_stats(g->stats, g->last)) return e;
         g->last.kernel_ms = ms;
         g->last.march_ms = mms;
-        g->last.rays = (int64_t)h[0];
-        g->last.steps = (int64_t)h[1];
-        g->last.capped = (int64_t)h[2];
-        g->last.bulk_slots = (int64_t)h[3];
-        g->last.bulk_steps = (int64_t)h[4];
         g->launched = false;
     }
     if (st) *st = g->last;

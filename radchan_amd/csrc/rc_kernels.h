@@ -154,6 +154,11 @@ void launch_finalize(hipStream_t st, const double *de, int n, int nVar, float *m
 /* de[u] = the compensated FP64 sum of ray[u photmax + h], h = 0..photmax-1,
  * in a fixed order (one wavefront per unit) */
 void launch_reduce_rays(hipStream_t st, const float *ray, size_t nunit, int photmax, double *de);
+/* the batched kernel's work queue: one counter per XCD's range, 256 bytes
+ * apart, so that requests to different counters do not queue up behind one
+ * another (a line takes about 90 per microsecond, all counters in one line
+ * 11 each); words of one launch's counters */
+constexpr int QPARTS = 8, QSTRIDE = 64, QUEUE_WORDS = QPARTS * QSTRIDE;
 /* workgroups of a batched launch over nunit_cells emitting (wall) cells,
  * and the 16-bit keys of radix-sort scratch it needs (0: none) */
 int batched_grid(const DevCommon &cm, long nunit_cells, int wg_per_cu);
@@ -162,6 +167,15 @@ int batched_grid(const DevCommon &cm, long nunit_cells, int wg_per_cu);
 void batched_schedule(const DevCommon &cm, int &wg_per_cu, int &threshold, int &spi, int &refill);
 size_t batched_srt_keys(const DevCommon &cm, long nunit_cells, int wg_per_cu);
 void launch_zero(hipStream_t st, double *p, size_t n);
+/* The solve's counters (rays, steps, capped, bulk slots, bulk steps) in
+ * STAT_LINES copies 256 bytes apart, a workgroup adding to the copy of its
+ * index: every wavefront adds its own, and one line takes about 90 adds per
+ * microsecond (8192 wavefronts on one line: 0.37 ms of a 16^3 solve).  The
+ * host sums them. */
+constexpr int STAT_LINES = 32, STAT_STRIDE = 32, STAT_WORDS = STAT_LINES * STAT_STRIDE;
+__device__ inline unsigned long long *stat_line(unsigned long long *stats) {
+    return stats + (blockIdx.x % STAT_LINES) * STAT_STRIDE;
+}
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n);
 /* k and Ib of every table row at each snapshot's Tmax, to its kbm, and the
  * quarter entries of its g CDFs, to its cdf_g4 */

@@ -326,8 +326,8 @@ __global__ void __launch_bounds__(128) k_fluid_plain(DevCommon cm, const DevSnap
         rays += __shfl_xor(rays, o);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stats[0], (unsigned long long)rays);
-        atomicAdd(&stats[1], (unsigned long long)steps);
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
+        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
     }
 }
 
@@ -367,8 +367,8 @@ __global__ void __launch_bounds__(128) k_fluid_band(DevCommon cm, const DevSnap 
         rays += __shfl_xor(rays, o);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stats[0], (unsigned long long)rays);
-        atomicAdd(&stats[1], (unsigned long long)steps);
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
+        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
     }
 }
 
@@ -408,8 +408,8 @@ __global__ void __launch_bounds__(128) k_surface_plain(DevCommon cm, const DevSn
         rays += __shfl_xor(rays, o);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stats[0], (unsigned long long)rays);
-        atomicAdd(&stats[1], (unsigned long long)steps);
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
+        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
     }
 }
 
@@ -444,8 +444,8 @@ k_fluid_f64(DevCommon cm, const DevSnap *__restrict__ snaps, int s, int v, const
         rays += __shfl_xor(rays, o);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stats[0], (unsigned long long)rays);
-        atomicAdd(&stats[1], (unsigned long long)steps);
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
+        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
     }
 }
 
@@ -475,8 +475,8 @@ k_surface_f64(DevCommon cm, const DevSnap *__restrict__ snaps, int s, int v, con
         rays += __shfl_xor(rays, o);
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stats[0], (unsigned long long)rays);
-        atomicAdd(&stats[1], (unsigned long long)steps);
+        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
+        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
     }
 }
 
