@@ -764,13 +764,14 @@ int rc_set_fields(rc_ctx *c, int nsnap, const float *const *T, int zstart) {
                  * positions); bd=4 z walls keep the texture mean */
                 const bool wx = (p.bd[FW] == 2 && p.adiabw == 1) || (p.bd[FE] == 2 && p.adiabe == 1);
                 const size_t nw = (size_t)2 * p.maxj[g] * p.maxk[g];
+                const size_t na = spline_axes_floats();
                 const size_t ns = spline_scratch_floats(p.imax, p.jmax, p.kmax, p.maxi[g], p.maxj[g], p.maxk[g]);
-                if (int e = c->spl.ensure((ns + nl + nw) * 4)) return e;
-                float *tl = c->spl.as<float>() + ns, *tw = tl + nl;
+                if (int e = c->spl.ensure((na + ns + nl + nw) * 4)) return e;
+                float *tl = c->spl.as<float>() + na + ns, *tw = tl + nl;
                 launch_spline_level(c->stream, S.T0.as<float>(), c->cx[0].as<float>(), c->cy[0].as<float>(),
                                     c->cz[0].as<float>(), c->cx[g].as<float>(), c->cy[g].as<float>(),
                                     c->cz[g].as<float>(), p.imax, p.jmax, p.kmax, p.maxi[g], p.maxj[g], p.maxk[g],
-                                    tl, wx ? tw : nullptr, c->spl.as<float>());
+                                    tl, wx ? tw : nullptr, c->spl.as<float>() + na, c->spl.as<float>());
                 launch_pos_from_T(c->stream, p, g, tl, wx ? tw : nullptr, tset.Tnb0, tset.invdT, p.nT, Pg, Tg);
             }
         }
@@ -1015,9 +1016,9 @@ int rc_spline_restrict(const rc_params *p, int level, const float *T, float *Tc,
     int rc = 0;
     {
         DevBuf dT, dc, dw, x0, y0, z0, xc, yc, zc, scr;
-        const size_t ns = spline_scratch_floats(p->imax, p->jmax, p->kmax, im, jm, km);
+        const size_t na = spline_axes_floats(), ns = spline_scratch_floats(p->imax, p->jmax, p->kmax, im, jm, km);
         if ((rc = dT.ensure(nT0 * 4)) || (rc = dc.ensure(nc * 4)) || (rc = dw.ensure(nw * 4)) ||
-            (rc = scr.ensure(ns * 4)) || (rc = upload(x0, g0.x, st)) || (rc = upload(y0, g0.y, st)) ||
+            (rc = scr.ensure((na + ns) * 4)) || (rc = upload(x0, g0.x, st)) || (rc = upload(y0, g0.y, st)) ||
             (rc = upload(z0, g0.z, st)) || (rc = upload(xc, gc.x, st)) || (rc = upload(yc, gc.y, st)) ||
             (rc = upload(zc, gc.z, st))) {
             (void)hipStreamSynchronize(st);
@@ -1028,7 +1029,7 @@ int rc_spline_restrict(const rc_params *p, int level, const float *T, float *Tc,
         if (e == hipSuccess) {
             launch_spline_level(st, dT.as<float>(), x0.as<float>(), y0.as<float>(), z0.as<float>(), xc.as<float>(),
                                 yc.as<float>(), zc.as<float>(), p->imax, p->jmax, p->kmax, im, jm, km, dc.as<float>(),
-                                Tw ? dw.as<float>() : nullptr, scr.as<float>());
+                                Tw ? dw.as<float>() : nullptr, scr.as<float>() + na, scr.as<float>());
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipMemcpyAsync(Tc, dc.p, nc * 4, hipMemcpyDeviceToHost, st);
