@@ -144,6 +144,8 @@ struct rc_ctx {
     DevBuf bacc;                            /* per-band plain variant: FP32 cell sums */
     int reduction = 0;                      /* batched tallies: 0 FP64 atomics, 1 deterministic */
     DevBuf rayf, rayw;                      /* deterministic reduction: per-ray tallies */
+    DevBuf ray64;                           /* FP64 path: per-ray tallies of one launch */
+    int runs64 = 1;                         /* and the runs they are of */
     DevBuf srtk;                            /* batched, srt above 256 keys: radix-sort scratch */
     DevBuf tr_rays, tr_unit, tr_ulist, tr_out;
     rc_stats last{};
@@ -804,7 +806,26 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
     launch_zero_u64(c->stream, c->stats.as<unsigned long long>(), STAT_WORDS);
     ++n;
     if (timed) RC_HIP(hipEventRecord(c->evm0, c->stream));
-    if (variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) {
+    if (p.fp64 == 1) {
+        /* as many runs at a time as rc_run found scratch for */
+        const size_t vk = (size_t)std::max(c->ncell, 2 * c->nsurf) * p.photmax;
+        for (int s = 0; s < nsnap; ++s)
+            for (int surface = 0; surface <= (walls ? 1 : 0); ++surface) {
+                const int nunit = surface ? 2 * c->nsurf : c->ncell;
+                double *out = surface ? c->ds.as<double>() + (size_t)s * nunit * p.nVar
+                                      : c->de.as<double>() + (size_t)s * nunit * p.nVar;
+                for (int v0 = 0; v0 < p.nVar; v0 += c->runs64) {
+                    const int nv = std::min(c->runs64, p.nVar - v0);
+                    uint16_t *keys = cm.srt ? c->keys.as<uint16_t>() : nullptr;
+                    for (int v = 0; cm.srt && v < nv; ++v) {
+                        launch_sort(c->stream, cm, ds, s, v0 + v, surface, nunit, nullptr, keys + v * vk);
+                        ++n;
+                    }
+                    n += launch_rays64(c->stream, cm, ds, s, v0, nv, surface, keys, vk, c->ray64.as<double>(),
+                                       c->ray64.bytes / 8, c->queue.as<int>(), out, c->stats.as<unsigned long long>());
+                }
+            }
+    } else if (variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) {
         for (int s = 0; s < nsnap; ++s) {
             double *de = c->de.as<double>() + (size_t)s * c->ncell * p.nVar;
             for (int v = 0; v < p.nVar; ++v) {
@@ -813,10 +834,6 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
                     launch_fluid_bands(c->stream, cm, ds, s, v, c->keys.as<uint16_t>(), c->bacc.as<float>(), de,
                                        c->stats.as<unsigned long long>());
                     n += p.nB + 2;
-                } else if (p.fp64 == 1) {
-                    launch_fluid_f64(c->stream, cm, ds, s, v, cm.srt ? c->keys.as<uint16_t>() : nullptr, de,
-                                     c->stats.as<unsigned long long>());
-                    ++n;
                 } else {
                     launch_fluid_plain(c->stream, cm, ds, s, v, cm.srt ? c->keys.as<uint16_t>() : nullptr, de,
                                        c->stats.as<unsigned long long>());
@@ -827,12 +844,8 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
                 double *dw = c->ds.as<double>() + (size_t)s * 2 * c->nsurf * p.nVar;
                 for (int v = 0; v < p.nVar; ++v) {
                     if (cm.srt) { launch_sort(c->stream, cm, ds, s, v, 1, 2 * c->nsurf, nullptr, c->keys.as<uint16_t>()); ++n; }
-                    if (p.fp64 == 1)
-                        launch_surface_f64(c->stream, cm, ds, s, v, cm.srt ? c->keys.as<uint16_t>() : nullptr, dw,
-                                           c->stats.as<unsigned long long>());
-                    else
-                        launch_surface_plain(c->stream, cm, ds, s, v, cm.srt ? c->keys.as<uint16_t>() : nullptr,
-                                             dw, c->stats.as<unsigned long long>());
+                    launch_surface_plain(c->stream, cm, ds, s, v, cm.srt ? c->keys.as<uint16_t>() : nullptr,
+                                         dw, c->stats.as<unsigned long long>());
                     ++n;
                 }
             }
@@ -896,8 +909,27 @@ int rc_run(rc_ctx *c, int variant) {
         set_error("the per-band plain variant needs sorted band keys (srt=1, narrow band)");
         return -2;
     }
+    if (p.fp64 == 1) {
+        /* tallies of every ray of all runs, at most 2 GiB, else as many as
+         * there is memory for (one unit's at least): the launches are split
+         * to fit */
+        const size_t P = (size_t)p.photmax, nr = (size_t)std::max(c->ncell, p.calcwalls == 1 ? 2 * c->nsurf : 0) * P;
+        size_t want = std::max(std::min(nr * p.nVar, (size_t)1 << 28), P);
+        while (!c->ray64.p) {
+            if (hipMalloc(&c->ray64.p, want * 8) == hipSuccess) { c->ray64.bytes = want * 8; break; }
+            c->ray64.p = nullptr;
+            (void)hipGetLastError();
+            if (want == P) { set_error("device allocation of " + std::to_string(want * 8) + " bytes failed"); return -11; }
+            want = std::max(want / 2, P);
+        }
+        c->runs64 = (int)std::max<size_t>(1, std::min<size_t>(p.nVar, c->ray64.bytes / 8 / nr));
+    }
     if ((variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) && p.srt == 1 && !p.grey) {
         const size_t nk = (size_t)std::max(c->ncell, 2 * c->nsurf) * p.photmax;
+        if (p.fp64 == 1 && c->runs64 > 1 && c->keys.ensure(nk * c->runs64 * 2) != 0) {
+            (void)hipGetLastError();
+            c->runs64 = 1;
+        }
         if (int e = c->keys.ensure(nk * 2)) return e;
     }
     if (variant == RC_VARIANT_PLAIN_BANDS)

@@ -144,12 +144,14 @@ void launch_fluid_bands(hipStream_t st, const DevCommon &cm, const DevSnap *snap
                         float *acc, double *de, unsigned long long *stats);
 void launch_surface_plain(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v,
                           const uint16_t *keys, double *de, unsigned long long *stats);
-/* the full-FP64 variant (floatpoint 1) in the plain launch shape: FP64
- * geometry, energy and cell sums; the snapshot's T_all must be set */
-void launch_fluid_f64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v, const uint16_t *keys,
-                      double *de, unsigned long long *stats);
-void launch_surface_f64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v,
-                        const uint16_t *keys, double *de, unsigned long long *stats);
+/* the full-FP64 variant (floatpoint 1): FP64 geometry, energy and sums (in
+ * ray order) of the fluid's (the walls') units in runs v0 .. v0 + nv - 1,
+ * whose keys are vkeys apart; the snapshot's T_all must be set.  ray: scratch
+ * of nray >= nv photmax tallies, worked through in as many launches as it takes;
+ * queue: QUEUE_WORDS words.  Returns the launch count. */
+int launch_rays64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v0, int nv, int surface,
+                  const uint16_t *keys, size_t vkeys, double *ray, size_t nray, int *queue, double *de,
+                  unsigned long long *stats);
 void launch_trace(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int surface, const int32_t *rays,
                   const int32_t *unit, int n, const uint16_t *keys, rc_ray *out);
 void launch_finalize(hipStream_t st, const double *de, int n, int nVar, float *mean, float *sdev);

@@ -414,69 +414,496 @@ __global__ void __launch_bounds__(128) k_surface_plain(DevCommon cm, const DevSn
 }
 
 /* ------------------------------------------------------------------------ */
-/* full-FP64 variant (floatpoint 1): the reference's launch shape, a thread  */
-/* per emitting (wall) cell, rays in sequence, FP64 per-cell sums.  Both     */
-/* kernels are held to 128 VGPRs (4 wavefronts per SIMD, a few spills): 7 %  */
-/* faster at 192x128x192 than with the 151 registers and 3 wavefronts they   */
-/* take unbounded.                                                          */
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_fluid_f64(DevCommon cm, const DevSnap *__restrict__ snaps, int s, int v, const uint16_t *__restrict__ keys,
-            double *__restrict__ de, unsigned long long *__restrict__ stats) {
-    const DevSnap &sn = snaps[s];
-    int64_t steps = 0, rays = 0;
-    for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < cm.ncell; n += gridDim.x * blockDim.x) {
-        int i, j, k;
-        cell_ijk(cm, n, i, j, k);
-        const uint32_t cid = (uint32_t)n + (uint32_t)cm.imax * cm.jmax * (cm.zstart - 1);
-        const float Ti = cell_T(cm, sn, i, j, k);
-        double acc = 0.0;
-        int st = 0;
-        for (int h = 0; h < cm.photmax; ++h) {
-            const uint32_t key = keys ? (uint32_t)keys[(size_t)n * cm.photmax + h] : 0u;
-            acc += fluid_ray64(cm, sn, i, j, k, cid, v, h, key, keys != nullptr, Ti, st);
-        }
-        steps += st;
-        rays += cm.photmax;
-        de[(size_t)n * cm.nVar + v] = acc;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        steps += __shfl_xor(steps, o);
-        rays += __shfl_xor(rays, o);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
-        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
-    }
+/* full-FP64 variant (floatpoint 1)                                          */
+
+/* generated rays of a wavefront */
+struct Rec64 {
+    double sx[64], sy[64], sz[64], isx[64], isy[64], isz[64], W[64], Bi[64], rBi[64];
+    float x[64], y[64], z[64];              /* the start is at single-precision coordinates */
+    int ic[64], jc[64], kc[64];
+    uint32_t row[64], id[64];
+};
+/* a ray being marched, handed from a lane to the whole wavefront */
+struct Drain64 {
+    double xp, yp, zp, sx, sy, sz, isx, isy, isz, tra, W, Bi, rBi, de;
+    int ic, jc, kc, cnt, g;
+    uint32_t row, id, pad;
+};
+/* LDS of coop64: factors or terms of the steps, transmissivities before them */
+struct Chain64 {
+    double x[64], tra[64];
+};
+/* rays left to a wavefront at which it stops marching them side by side */
+constexpr int COOP64 = 8;
+struct Lev64 {
+    const float *xu, *T;
+    int im, jm, km, maxs;
+    float dy, dz;
+};
+__device__ __forceinline__ Lev64 lev64(const DevSnap &sn, int g) {
+    const DevLevel &L = sn.lev[g];
+    return Lev64{L.xu, sn.T_all + L.poff, L.im, L.jm, L.km, L.maxs, L.dy, L.dz};
 }
 
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_surface_f64(DevCommon cm, const DevSnap *__restrict__ snaps, int s, int v, const uint16_t *__restrict__ keys,
-              double *__restrict__ de, unsigned long long *__restrict__ stats) {
-    const DevSnap &sn = snaps[s];
-    int64_t steps = 0, rays = 0;
-    for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < 2 * cm.nsurf; n += gridDim.x * blockDim.x) {
-        const int bound = n / cm.nsurf, w = n % cm.nsurf;
-        if (!cm.adiab[bound]) continue;
-        const int j = w % cm.jmax + 1, k = w / cm.jmax + cm.zstart;
-        const uint32_t cid = (uint32_t)(w + cm.jmax * (cm.zstart - 1));
-        const float Tw = wall_T(cm, sn, bound, j, k);
-        double acc = 0.0;
-        int st = 0;
-        for (int h = 0; h < cm.photmax; ++h) {
-            const uint32_t key = keys ? (uint32_t)keys[(size_t)n * cm.photmax + h] : 0u;
-            acc += surface_ray64(cm, sn, bound, j, k, cid, v, h, key, keys != nullptr, Tw, st);
+/* LDS written by some lanes of the wavefront, then read by others */
+__device__ __forceinline__ void wave_lds64() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+/* x of another lane of the quad (a DPP quad_perm) */
+template <int PERM>
+__device__ __forceinline__ double quad64(double x) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    return bits2d(((uint64_t)(uint32_t)__builtin_amdgcn_mov_dpp((int)(b >> 32), PERM, 0xF, 0xF, true) << 32) |
+                  (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, PERM, 0xF, 0xF, true));
+}
+
+/* what a ray that leaves the grid through `face` (no periodic or specular
+ * one) is tallied: a black wall's emission, from a fixed temperature's Ib
+ * (the row's entry of the face) or the table at the wall's temperature
+ * (adiabatic x walls, bd 4 z walls); nothing if lost */
+__device__ __forceinline__ double wall64(const DevCommon &cm, const DevSnap &sn, const Lev64 &L, uint32_t row, int face,
+                                         const Ray &r, double W, double tra, double Bi, double rBi) {
+    const int bd = cm.bd[face];
+    if (bd != 2 && bd != 4) return 0.0;
+    double Bw;
+    if ((face == FW && cm.adiab[0]) || (face == FE && cm.adiab[1]) || bd == 4) {
+        double Kw;
+        kb64(sn, sn.kb + row, cm.nT, (double)gld(L.T, wall_index(L, r, face)), Kw, Bw);
+    } else {
+        Bw = (double)gld(sn.kb, row + (uint32_t)(cm.nT + 1 + 2 * face)).y;
+    }
+    return W * tra * excess64(Bw, Bi, rBi);
+}
+/* indices on level g + 1 of those on level g (:215-223) */
+__device__ __forceinline__ void coarsen64(const DevSnap &sn, int g, int &ic, int &jc, int &kc) {
+    const DevLevel &L = sn.lev[g], &M = sn.lev[g + 1];
+    const int ri = L.im / M.im, rj = L.jm / M.jm, rk = L.km / M.km;
+    ic = (ic + ri - 1) / ri;
+    jc = (jc + rj - 1) / rj;
+    kc = (kc + rk - 1) / rk;
+}
+
+/* Units u0 .. u0 + nu - 1 (fluid cells, or wall cells of both walls) in runs
+ * run0 .. run0 + nv - 1, run v's keys at keys + (v - run0) vkeys: ray q's
+ * tally to ray[q], q = ((v - run0) nu + unit) photmax + h, for k_sum_rays64
+ * to add up in ray order, which is the sum of a thread that traces its
+ * cell's rays in turn, to the bit.  Free of that order, a wavefront takes
+ * ranges of rays off a queue (one counter per XCD, as the batched kernel's),
+ * generates them 64 at a time into LDS and has its lanes take the next
+ * whenever REFILL64 of them are idle; its last COOP64 rays it marches
+ * together (coop64).  (MG: several levels.)
+ *
+ * 64^3, 100 rays, 2 runs (302 M steps, the longest ray 21 000): a thread per
+ * cell, its wavefront waiting for the longest of 64 rays and at last for
+ * the longest of all, took 2 x 17.3 ms; both runs in one launch now take 8.1
+ * ms, of which 4.6 are the bulk (FP64 arithmetic, about 150 instructions per
+ * step) and the rest the last rays: a lone lane's step takes about 3000
+ * clocks, coop64's 430 (15.3 ms per run without it).  REFILL64 4 to 16 and
+ * STEPS64 1 to 4 are within 5 %; COOP64 4 to 16 within 1 %; 3 wavefronts per
+ * SIMD instead of 4 (128 registers, a few spills) 2 % slower; stopping the
+ * wavefront for a ray of over 1000 steps to march it together at once, the
+ * same. */
+constexpr int REFILL64 = 8, STEPS64 = 2;
+static_assert(COOP64 * sizeof(Drain64) + sizeof(Chain64) <= sizeof(Rec64), "the drain's LDS");
+
+__device__ __forceinline__ int uni64(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ double lane64(double x, int l) {
+    const uint64_t b = (uint64_t)__double_as_longlong(x);
+    return bits2d(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(b >> 32), l) << 32) |
+                  (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l));
+}
+
+/* The rest of one ray by the whole wavefront, 64 steps at a time: the
+ * geometry, which is serial, lane 4 q + a the axis a (every quad the same),
+ * lane n keeping step n's cell and path; then table, exponential and excess
+ * of all steps at once; then the transmissivities and the tally in step
+ * order by one lane.  The operations on the ray are those of the loop in
+ * k_rays64.  Returns the steps. */
+template <bool MG>
+__device__ int coop64(const DevCommon &cm, const DevSnap &sn, const Drain64 &r, uint32_t bds, double tl, Chain64 &ch,
+                      double &de_out) {
+    const int lane = threadIdx.x & 63, a = lane & 3;
+    const double W = r.W, Bi = r.Bi, rBi = r.rBi;
+    double tra = r.tra, de = r.de;
+    /* the axis' position and direction; lane 3 of a quad is never crossed
+     * (its face, position and direction stay 1e300, 0, 0 and 1) */
+    double p = a == 0 ? r.xp : (a == 1 ? r.yp : (a == 2 ? r.zp : 0.0));
+    double s = a == 0 ? r.sx : (a == 1 ? r.sy : (a == 2 ? r.sz : 0.0));
+    double is = a == 0 ? r.isx : (a == 1 ? r.isy : (a == 2 ? r.isz : 1.0));
+    int cnt = uni64(r.cnt), g = MG ? uni64(r.g) : 0, steps = 0;
+    const uint32_t row = (uint32_t)uni64((int)r.row);
+    Lev64 L = lev64(sn, g);
+    /* the axis' next face j of 0..nf and its coordinate f, the unit step u,
+     * cells stride apart */
+    int j, nf, u, stride;
+    float dyz;
+    double f;
+    uint32_t c;                                         /* the cell (uniform) */
+    auto level = [&](int ic, int jc, int kc) {
+        nf = a == 0 ? L.im : (a == 1 ? L.jm : L.km);
+        stride = a == 0 ? 1 : (a == 1 ? L.im : L.im * L.jm);
+        dyz = a == 1 ? L.dy : L.dz;
+        u = s < 0.0 ? -1 : 1;
+        j = (a == 0 ? ic : (a == 1 ? jc : kc)) - (s < 0.0 ? 1 : 0);
+        c = (uint32_t)(ic - 1) + (uint32_t)L.im * ((uint32_t)(jc - 1) + (uint32_t)L.jm * (uint32_t)(kc - 1));
+    };
+    auto xface = [&](int q) { return gld32(L.xu, (uint32_t)min(max(q, 0), L.im)); };
+    auto index = [&](int axis) { return __builtin_amdgcn_readlane(j + (s < 0.0 ? 1 : 0), axis); };
+    level(uni64(r.ic), uni64(r.jc), uni64(r.kc));
+    for (;;) {
+        int n = 0, end = -1;
+        double pds = 0.0;
+        uint32_t pc = 0;
+        const int cap = min(64, L.maxs - cnt);
+        while (n < cap && end < 0) {
+            /* (re)entered after a boundary */
+            const int last = s < 0.0 ? 0 : nf, du = u * stride;
+            float xn = xface(j + u);                    /* the x face after the next */
+            f = a == 0 ? (double)xface(j) : (a == 3 ? 1e300 : (double)((float)j * dyz));
+            int ax;
+            bool ev;
+            do {
+                const double d = (f - p) * is;
+                double m = d, o = quad64<0xB1>(d);
+                m = o < m ? o : m;
+                o = quad64<0x4E>(m);
+                m = o < m ? o : m;
+                /* the tie rules: z before y before x (and z if nothing compares) */
+                ax = (0xAA52 >> (2 * (int)(__ballot(d == m) & 7ull))) & 3;
+                const bool cr = a == ax;
+                ev = (__ballot(j == last) & (7ull & (1ull << ax))) != 0ull;
+                if (lane == n) { pds = m; pc = c; }
+                ++n;
+                p = (d == m) ? f : fma(m, s, p);
+                j += cr ? u : 0;
+                const double fn = a == 0 ? (double)xn : (double)((float)j * dyz);
+                f = cr ? fn : f;
+                c += (uint32_t)__builtin_amdgcn_readlane(du, ax);
+                if (ax == 0) xn = xface(j + u);
+            } while (!ev && n < cap);
+            if (!ev) break;
+            const int d = __builtin_amdgcn_readlane(s < 0.0 ? 1 : 0, ax), face = 2 * ax + 1 - d;
+            const int bd = (int)(bds >> (4 * face)) & 15;
+            if (bd == 1 || bd == 3) {                             /* periodic, specular: on from one of the sides */
+                const bool hi = (d != 0) == (bd == 1);
+                if (a == ax) {
+                    p = hi ? (double)(a == 0 ? cm.Lx : (a == 1 ? cm.Ly : cm.Lz)) : 0.0;
+                    if (bd == 3) { s = -s; is = -is; u = s < 0.0 ? -1 : 1; }
+                    j = (hi ? nf : 1) - (s < 0.0 ? 1 : 0);
+                }
+                const int ic = index(0), jc = index(1), kc = index(2);
+                c = (uint32_t)(ic - 1) + (uint32_t)L.im * ((uint32_t)(jc - 1) + (uint32_t)L.jm * (uint32_t)(kc - 1));
+            } else {
+                end = face;
+            }
         }
-        steps += st;
-        rays += cm.photmax;
-        de[(size_t)n * cm.nVar + v] = acc;
+        /* attenuation of the block's steps (:358-370) */
+        double em = 0.0, ex = 1.0, fac = 0.0;
+        if (lane < n) {
+            int t;
+            double al;
+            pos64(sn, cm.nT, (double)gld(L.T, pc), t, al);
+            const float2 v0 = gld(sn.kb, row + t), v1 = gld(sn.kb, row + t + 1);
+            const double K = lerp64(v0.x, v1.x, al), B = lerp64(v0.y, v1.y, al), x = K * pds;
+            fac = excess64(B, Bi, rBi);
+            expm1_exp_d(-x, em, ex);
+        }
+        ch.x[lane] = ex;                                /* (1 beyond n) */
+        wave_lds64();
+        if (lane == 0)
+            for (int k = 0; k < n; k += 8) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    ch.tra[k + q] = tra;
+                    tra = tra * ch.x[k + q];
+                }
+            }
+        wave_lds64();
+        const double trb = ch.tra[lane], tral = trb * ex, lastt = W * tral * fac;
+        const unsigned long long stop = __ballot(lane < n && !(tral > tl));
+        const int m = stop ? (int)__builtin_ctzll(stop) + 1 : n;
+        ch.x[lane] = lane < m ? W * trb * (-em) * fac : 0.0;
+        wave_lds64();
+        if (lane == 0)
+            for (int k = 0; k < m; k += 8) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) de -= ch.x[k + q];
+            }
+        wave_lds64();
+        de = lane64(de, 0);
+        tra = lane64(tra, 0);
+        if (stop) {
+            tra = lane64(tral, m - 1);
+            if (tra < tl) {
+                de -= lane64(lastt, m - 1);
+                tra = 0.0;
+            }
+        }
+        steps += m;
+        cnt += m;
+        if (m == n && end >= 0) {
+            const Ray rr{index(0), index(1), index(2), 0, 0, 0};
+            de -= wall64(cm, sn, L, row, end, rr, W, tra, Bi, rBi);
+            break;
+        }
+        if (stop) break;
+        if (cnt >= L.maxs) {
+            if (!MG || g >= cm.grid_num - 1) break;
+            int ic = index(0), jc = index(1), kc = index(2);
+            coarsen64(sn, g, ic, jc, kc);
+            g += 1;
+            cnt = 0;
+            L = lev64(sn, g);
+            level(ic, jc, kc);
+        }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        steps += __shfl_xor(steps, o);
-        rays += __shfl_xor(rays, o);
+    de_out = de;
+    return steps;
+}
+
+template <bool SURF, bool MG>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_rays64(DevCommon cm, const DevSnap *__restrict__ snaps, int s, int run0, int nv, const uint16_t *__restrict__ keys,
+         size_t vkeys, int u0, int nu, int *__restrict__ queue, double *__restrict__ ray,
+         unsigned long long *__restrict__ stats) {
+    __shared__ Rec64 recs[4];
+    const DevSnap &sn = snaps[s];
+    const int lane = threadIdx.x & 63;
+    Rec64 &q = recs[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    const uint32_t P = (uint32_t)cm.photmax, total = (uint32_t)nv * (uint32_t)nu * P;
+    const double tl = (double)(SURF ? cm.tollS : cm.toll);
+    const Lev64 L0 = lev64(sn, 0);
+    uint32_t bds = 0;                       /* 4 bits per face */
+#pragma unroll
+    for (int f = 0; f < 6; ++f) bds |= (uint32_t)cm.bd[f] << (4 * f);
+
+    /* wavefront state: the queue's range, the generated rays */
+    const int pwaves = max((int)gridDim.x * 4 / QPARTS, 1);
+    int part = (int)(blockIdx.x % QPARTS), ptries = 0, plast = 0;
+    uint32_t gpos = 0, gend = 0;
+    int qn = 0, qh = 0;
+    unsigned long long live = 0ull;
+    int64_t steps = 0;
+
+    /* lane state */
+    bool alive = false;
+    int ic = 1, jc = 1, kc = 1, cnt = 0, g = 0, f0 = 0, f1 = 0, f2 = 0, t = 0;
+    double xp = 0, yp = 0, zp = 0, sx = 0, sy = 0, sz = 0, isx = 0, isy = 0, isz = 0, tra = 0, W = 0, Bi = 1, rBi = 1,
+           de = 0, ta = 0;
+    uint32_t row = 0, id = 0;
+    float fxn = 0.f;
+    float2 v0 = make_float2(0.f, 0.f), v1 = v0;
+    Lev64 L = L0;
+
+    /* the cell's temperature and the x face ahead, then its table entries */
+    auto cell = [&]() {
+        fxn = gld(L.xu, (uint32_t)(ic - f0));
+        return gld(L.T, (uint32_t)(ic - 1) + (uint32_t)L.im * ((uint32_t)(jc - 1) + (uint32_t)L.jm * (uint32_t)(kc - 1)));
+    };
+    auto entries = [&](float T) {
+        pos64(sn, cm.nT, (double)T, t, ta);
+        v0 = gld(sn.kb, row + (uint32_t)t);
+        v1 = gld(sn.kb, row + (uint32_t)t + 1u);
+    };
+
+    for (;;) {
+        const int idle = 64 - __popcll(live);
+        if (idle >= REFILL64) {
+            if (qn == 0 && part >= 0) {
+                while (gpos >= gend && part >= 0) {
+                    const uint32_t pb = (uint32_t)((uint64_t)total * part / QPARTS);
+                    const uint32_t pe = (uint32_t)((uint64_t)total * (part + 1) / QPARTS);
+                    const int ask = min(max((int)((pe - pb) - plast) / (2 * pwaves), 64), 1024) & ~63;
+                    int c0 = 0;
+                    if (lane == 0) {
+                        if (ptries) c0 = __hip_atomic_load(&queue[part * QSTRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if ((uint32_t)c0 < pe - pb) c0 = atomicAdd(&queue[part * QSTRIDE], ask);
+                    }
+                    c0 = __builtin_amdgcn_readfirstlane(c0);
+                    if ((uint32_t)c0 < pe - pb) {
+                        plast = c0 + ask;
+                        gpos = pb + c0;
+                        gend = min(gpos + ask, pe);
+                    } else {
+                        part = (part + 1) % QPARTS;
+                        plast = 0;
+                        if (++ptries >= QPARTS) part = -1;
+                    }
+                }
+                if (gpos < gend) {
+                    qn = (int)min(gend - gpos, 64u);
+                    qh = 0;
+                    if (lane < qn) {
+                        const uint32_t x = gpos + lane, un = x / P, vi = un / (uint32_t)nu;
+                        const int v = run0 + (int)vi, n = u0 + (int)(un - vi * (uint32_t)nu);
+                        const int h = (int)(x - un * P);
+                        const uint32_t key = keys ? (uint32_t)keys[vi * vkeys + (size_t)n * P + h] : 0u;
+                        Ray64 r;
+                        En64 e;
+                        if (SURF) {
+                            const int bound = n / cm.nsurf, w = n % cm.nsurf;
+                            const int j = w % cm.jmax + 1, k = w / cm.jmax + cm.zstart;
+                            const uint32_t cid = (uint32_t)(w + cm.jmax * (cm.zstart - 1));
+                            surface_setup64(cm, sn, bound, j, k, cid, v, h, key, keys != nullptr,
+                                            wall_T(cm, sn, bound, j, k), r, e);
+                        } else {
+                            int i, j, k;
+                            cell_ijk(cm, n, i, j, k);
+                            const uint32_t cid = (uint32_t)n + (uint32_t)cm.imax * cm.jmax * (cm.zstart - 1);
+                            fluid_setup64(cm, sn, i, j, k, cid, v, h, key, keys != nullptr, cell_T(cm, sn, i, j, k), r, e);
+                        }
+                        q.sx[lane] = r.sx; q.sy[lane] = r.sy; q.sz[lane] = r.sz;
+                        q.isx[lane] = r.isx; q.isy[lane] = r.isy; q.isz[lane] = r.isz;
+                        q.x[lane] = (float)r.xp; q.y[lane] = (float)r.yp; q.z[lane] = (float)r.zp;
+                        q.W[lane] = e.W; q.Bi[lane] = e.Bi; q.rBi[lane] = e.rBi;
+                        q.ic[lane] = r.ic; q.jc[lane] = r.jc; q.kc[lane] = r.kc;
+                        q.row[lane] = e.row; q.id[lane] = x;
+                    }
+                    gpos += qn;
+                    wave_lds64();
+                }
+            }
+            if (qn) {
+                const int o = __builtin_amdgcn_mbcnt_hi((uint32_t)(~live >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)~live, 0u));
+                if (!alive && o < qn) {
+                    const int w = qh + o;
+                    sx = q.sx[w]; sy = q.sy[w]; sz = q.sz[w];
+                    isx = q.isx[w]; isy = q.isy[w]; isz = q.isz[w];
+                    xp = (double)q.x[w]; yp = (double)q.y[w]; zp = (double)q.z[w];
+                    W = q.W[w]; Bi = q.Bi[w]; rBi = q.rBi[w];
+                    ic = q.ic[w]; jc = q.jc[w]; kc = q.kc[w];
+                    row = q.row[w]; id = q.id[w];
+                    f0 = sx < 0.0; f1 = sy < 0.0; f2 = sz < 0.0;
+                    tra = 1.0;
+                    de = 0.0;
+                    cnt = 0;
+                    alive = true;                           /* (toll < 1) */
+                    if (MG) { g = 0; L = L0; }
+                    entries(cell());
+                }
+                const int took = min(idle, qn);
+                qn -= took;
+                qh += took;
+                wave_lds64();
+            } else if (64 - idle <= COOP64) {
+                break;
+            }
+        }
+        for (int k = 0; k < STEPS64; ++k) {
+            live = __ballot(alive);
+            steps += __popcll(live);
+            if (!alive) continue;
+            /* one step of march_ray (one iteration of the loop at
+             * mc_gpu_noint.cu:252-654) */
+            const double fx = (double)fxn;
+            const double fy = (double)((float)(jc - f1) * L.dy);
+            const double fz = (double)((float)(kc - f2) * L.dz);
+            const double dsx = (fx - xp) * isx, dsy = (fy - yp) * isy, dsz = (fz - zp) * isz;
+            double ds = dsx;
+            if (ds > dsy) ds = dsy;
+            if (ds > dsz) ds = dsz;
+            xp = (ds == dsx) ? fx : fma(ds, sx, xp);
+            yp = (ds == dsy) ? fy : fma(ds, sy, yp);
+            zp = (ds == dsz) ? fz : fma(ds, sz, zp);
+            /* one index along the crossed axis, with the tie rules */
+            const bool cx = dsx < dsy && dsx < dsz, cy = !(dsx < dsy) && dsy < dsz;
+            const int d = cx ? f0 : (cy ? f1 : f2);
+            ic += cx ? 1 - 2 * d : 0;
+            jc += cy ? 1 - 2 * d : 0;
+            kc += (cx || cy) ? 0 : 1 - 2 * d;
+            const uint32_t at = (uint32_t)(cx ? ic : (cy ? jc : kc)) - 1u, lim = (uint32_t)(cx ? L.im : (cy ? L.jm : L.km));
+            int end = -1;                           /* the face the ray ends at */
+            if (at >= lim) {
+                const int face = (cx ? FW : (cy ? FS : FB)) + (d ? 0 : 1);
+                const int bd = (int)(bds >> (4 * face)) & 15;
+                if (bd == 1 || bd == 3) {                         /* periodic, specular: on from one of the sides */
+                    const bool hi = (d != 0) == (bd == 1);
+                    const int ni = hi ? (int)lim : 1;
+                    const double np = hi ? (double)(cx ? cm.Lx : (cy ? cm.Ly : cm.Lz)) : 0.0;
+                    ic = cx ? ni : ic;
+                    jc = cy ? ni : jc;
+                    kc = (cx || cy) ? kc : ni;
+                    xp = cx ? np : xp;
+                    yp = cy ? np : yp;
+                    zp = (cx || cy) ? zp : np;
+                    if (bd == 3) {
+                        if (cx) { sx = -sx; isx = -isx; f0 = sx < 0.0; }
+                        else if (cy) { sy = -sy; isy = -isy; f1 = sy < 0.0; }
+                        else { sz = -sz; isz = -isz; f2 = sz < 0.0; }
+                    }
+                } else {
+                    end = face;
+                }
+            }
+            const float2 w0 = v0, w1 = v1;
+            const double wa = ta;
+            float Tn = 0.f;
+            if (end < 0) Tn = cell();
+            /* attenuation and the reciprocity tally (:358-370) */
+            const double K = lerp64(w0.x, w1.x, wa), B = lerp64(w0.y, w1.y, wa);
+            const double x = K * ds, fac = excess64(B, Bi, rBi);
+            double em, ex;
+            expm1_exp_d(-x, em, ex);
+            const double wta = W * tra * (-em);
+            de -= wta * fac;
+            tra = tra * ex;
+            if (tra < tl) {
+                de -= W * tra * fac;
+                tra = 0.0;
+            }
+            if (end >= 0) {
+                de -= wall64(cm, sn, L, row, end, Ray{ic, jc, kc, f0, f1, f2}, W, tra, Bi, rBi);
+                tra = 0.0;
+            }
+            cnt += 1;
+            alive = tra > tl;
+            if (cnt >= L.maxs && alive) {
+                /* still alive after the level's cap (:210-224): on to the
+                 * next level, indices coarsened (:215-223) */
+                alive = MG && g < cm.grid_num - 1;
+                if (alive) {
+                    coarsen64(sn, g, ic, jc, kc);
+                    g += 1;
+                    cnt = 0;
+                    L = lev64(sn, g);
+                    Tn = cell();
+                }
+            }
+            if (alive) entries(Tn);
+            else ray[id] = de;
+        }
+        live = __ballot(alive);
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&stat_line(stats)[0], (unsigned long long)rays);
-        atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
+    /* nothing left to generate and few rays marching: one after the other */
+    Drain64 *dr = reinterpret_cast<Drain64 *>(&q);
+    Chain64 &ch = *reinterpret_cast<Chain64 *>(dr + COOP64);
+    if (alive) {
+        const int o = __builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0u));
+        dr[o] = Drain64{xp, yp, zp, sx, sy, sz, isx, isy, isz, tra, W, Bi, rBi, de, ic, jc, kc, cnt, g, row, id, 0u};
+    }
+    wave_lds64();
+    const int nd = __popcll(live);
+    for (int o = 0; o < nd; ++o) {
+        double sum;
+        steps += coop64<MG>(cm, sn, dr[o], bds, tl, ch, sum);
+        if (lane == 0) ray[dr[o].id] = sum;
+    }
+    if (lane == 0) atomicAdd(&stat_line(stats)[1], (unsigned long long)steps);
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&stat_line(stats)[0], (unsigned long long)total);
+}
+
+/* each (unit, run)'s tallies added in ray order */
+__global__ void __launch_bounds__(128) k_sum_rays64(const double *__restrict__ ray, int u0, int nu, int P, int nVar,
+                                                    int run0, int nv, double *__restrict__ de) {
+    for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < nv * nu; w += gridDim.x * blockDim.x) {
+        const int vi = w / nu, n = w - vi * nu;
+        const double *r = ray + (size_t)w * P;
+        double acc = 0.0;
+#pragma unroll 8
+        for (int h = 0; h < P; ++h) acc += r[h];
+        de[(size_t)(u0 + n) * nVar + run0 + vi] = acc;
     }
 }
 
@@ -624,16 +1051,28 @@ void launch_field_scan(hipStream_t st, const float *T, int imax, int jmax, int k
     hipLaunchKernelGGL(k_field_scan, dim3(blocks), dim3(256), 0, st, T, imax, jmax, kmax, out);
 }
 
-void launch_fluid_f64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v, const uint16_t *keys,
-                      double *de, unsigned long long *stats) {
-    const int blocks = std::max(1, std::min((cm.ncell + 127) / 128, 1 << 20));
-    hipLaunchKernelGGL(k_fluid_f64, dim3(blocks), dim3(128), 0, st, cm, snaps, s, v, keys, de, stats);
-}
-
-void launch_surface_f64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v,
-                        const uint16_t *keys, double *de, unsigned long long *stats) {
-    const int blocks = std::max(1, std::min((2 * cm.nsurf + 127) / 128, 1 << 20));
-    hipLaunchKernelGGL(k_surface_f64, dim3(blocks), dim3(128), 0, st, cm, snaps, s, v, keys, de, stats);
+int launch_rays64(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int s, int v0, int nv, int surface,
+                  const uint16_t *keys, size_t vkeys, double *ray, size_t nray, int *queue, double *de,
+                  unsigned long long *stats) {
+    const int ub = surface ? (cm.adiab[0] ? 0 : cm.nsurf) : 0;
+    const int ue = surface ? (cm.adiab[1] ? 2 * cm.nsurf : cm.nsurf) : cm.ncell;
+    const size_t P = (size_t)cm.photmax;
+    int n = 0;
+    for (int u = ub, nu = 0; u < ue; u += nu) {
+        nu = (int)std::max<size_t>(1, std::min<size_t>(nray / nv / P, (size_t)(ue - u)));
+        const int blocks = (int)std::min<size_t>((nv * nu * P + 255) / 256, 4 * 256);
+        launch_zero_u64(st, reinterpret_cast<unsigned long long *>(queue), QUEUE_WORDS / 2);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, st, cm, snaps, s, v0, nv, keys, vkeys, u, nu, queue, ray,
+                               stats);
+        };
+        if (surface) { if (cm.grid_num > 1) go(k_rays64<true, true>); else go(k_rays64<true, false>); }
+        else { if (cm.grid_num > 1) go(k_rays64<false, true>); else go(k_rays64<false, false>); }
+        const int sb = (int)std::min<size_t>(((size_t)nv * nu + 127) / 128, 1 << 20);
+        hipLaunchKernelGGL(k_sum_rays64, dim3(sb), dim3(128), 0, st, ray, u, nu, cm.photmax, cm.nVar, v0, nv, de);
+        n += 3;
+    }
+    return n;
 }
 
 void launch_trace(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int surface, const int32_t *rays,
