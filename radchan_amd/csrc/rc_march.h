@@ -436,6 +436,10 @@ __device__ __forceinline__ void march_ahead(const DevCommon &cm, const S &sn, co
 
 /* x of another lane of the quad (a DPP quad_perm) */
 template <int PERM>
+__device__ __forceinline__ int quad_lane(int x) {
+    return __builtin_amdgcn_mov_dpp(x, PERM, 0xF, 0xF, true);
+}
+template <int PERM>
 __device__ __forceinline__ float quad_lane(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), PERM, 0xF, 0xF, true));
 }
@@ -453,9 +457,13 @@ __device__ __forceinline__ float quad_lane(float x) {
  * and in the same order, so the tally, transmissivity and step count are
  * bit-identical to it.  Returns at the ray's end or at the level's step
  * cap; expects a live ray under the cap.  `xul`: the level's x faces in
- * LDS.  A lone wavefront issues an instruction every 7 clocks or so: with
- * all three axes in every lane a step took 600 clocks, now 420
- * (64^3, whose longest ray has 21 000 steps: march 9.8 -> 8.2 ms). */
+ * LDS.  Bound by the step's chain of dependent instructions, and by its
+ * branches where they are taken (all but the loop's own are to code out of
+ * line; with the events in an outer loop the same step took longer than
+ * with half as many instructions again): all three axes in every lane
+ * 600 clocks a step, an axis per lane 420, the next face and its successor
+ * kept ready 380.  64^3, whose longest ray has 21 000 steps: march 9.8, 8.1
+ * and 7.8 ms. */
 template <int TM, class S>
 __device__ __forceinline__ void march_coop(const DevCommon &cm, const S &sn, const DevLevel &L, const Ray &r,
                                            const En &e, float tol, float &de, int &counter, int &nsteps,
@@ -470,64 +478,87 @@ __device__ __forceinline__ void march_coop(const DevCommon &cm, const S &sn, con
     const int nf = a == 0 ? L.im : (a == 1 ? L.jm : L.km), stride = a == 0 ? 1 : (a == 1 ? L.im : L.im * L.jm);
     const float dyz = a == 1 ? L.dy : L.dz;
     auto neg = [&]() { return s < 0.f ? 1 : 0; };
-    /* the axis' next face j of 0..nf (its cell index is j + neg()) */
-    int j = (a == 0 ? r.ic : (a == 1 ? r.jc : r.kc)) - neg();
-    auto index = [&](int axis) { return __builtin_amdgcn_readlane(j + neg(), axis); };
+    /* What a step needs first is ready before it: the face ahead, f, and the
+     * one after it, fn (index jn, as a float; past: its value once the grid
+     * is left, lane 3: none; xn: the x axis').  u: the axis' index step, cs
+     * its share of the cell index and du the share's step. */
+    float f, fn, xn, jn, past, uf;
+    int u, du, cs;
     auto xface = [&](int q) { return xul[min(max(q, 0), L.im)]; };
+    auto enter = [&](int ci) {                  /* from the axis' cell index */
+        const int j = ci - neg();
+        u = 1 - 2 * neg();
+        uf = (float)u;
+        du = a == 3 ? 0 : u * stride;
+        cs = a == 3 ? 0 : (ci - 1) * stride;
+        past = a == 3 ? -9.f : (neg() ? -2.f : (float)(nf + 2));
+        jn = (float)(j + u);
+        f = a == 0 ? xface(j) : (a == 3 ? 1e30f : (float)j * dyz);
+        xn = xface(j + u);
+        fn = a == 0 ? xn : jn * dyz;
+    };
+    enter(a == 0 ? r.ic : (a == 1 ? r.jc : r.kc));
+    float low = -INFINITY;
+    asm volatile("" : "+v"(low));       /* a median with -inf stays one: no quieting of its operands */
     for (;;) {
         uint32_t mcell = 0u;
         float mds = 0.f, wl = 0.f;
         int bl = RB_ON;
-        const int nmax = min(64, L.maxs - __builtin_amdgcn_readfirstlane(counter));
+        int nmax = min(64, L.maxs - __builtin_amdgcn_readfirstlane(counter));
         int n = 0;
-        while (n < nmax && bl == RB_ON) {
-            /* (re)entered after a face of the grid: unit step, the grid's
-             * face ahead, the step of the linear cell index, the cell, the
-             * faces ahead */
-            const int u = 1 - 2 * neg(), last = neg() ? 0 : nf, du = u * stride;
-            uint32_t cur = (uint32_t)(index(0) - 1) +
-                           (uint32_t)L.im * ((uint32_t)(index(1) - 1) + (uint32_t)L.jm * (uint32_t)(index(2) - 1));
-            float f = a == 0 ? xface(j) : (a == 3 ? 1e30f : (float)j * dyz);
-            float xn = xface(j + u);
-            int ax;
-            bool out;
-            do {
-                const float d = (f - p) * is;
-                float ds = __builtin_amdgcn_fmed3f(d, quad_lane<0xB1>(d), -INFINITY);
-                ds = __builtin_amdgcn_fmed3f(ds, quad_lane<0x4E>(ds), -INFINITY);
-                /* the axis crossed by the tie rules, z before y before x (z
-                 * if nothing compares) */
-                ax = (0xAA52 >> (2 * (int)(__ballot(d == ds) & 7ull))) & 3;
+        do {
+            const float d = (f - p) * is;
+            float ds = __builtin_amdgcn_fmed3f(d, quad_lane<0xB1>(d), low);
+            ds = __builtin_amdgcn_fmed3f(ds, quad_lane<0x4E>(ds), low);
+            const bool eq = d == ds;
+            const int ea = (int)__ballot(eq) & 7;
+            const float fo = f, pm = fmaf(ds, s, p);
+            f = eq ? fn : f;
+            p = eq ? fo : pm;
+            const int cq = cs + quad_lane<0xB1>(cs);
+            const int cur = cq + quad_lane<0x4E>(cq);
+            mcell = lane == n ? (uint32_t)cur : mcell;
+            mds = lane == n ? ds : mds;
+            n += 1;
+            jn += eq ? uf : 0.f;
+            cs += eq ? du : 0;
+            if (__builtin_expect(((0x14 >> ea) & 1) == 0, 0)) {
+                /* x crossed, or faces of several axes at once: the tie
+                 * rules, z before y before x (z if nothing compares) */
+                const int ax = (0xAA52 >> (2 * ea)) & 3;
                 const bool cr = a == ax;
-                out = (__ballot(j == last) & (7ull & (1ull << ax))) != 0ull;
-                mcell = lane == n ? cur : mcell;
-                mds = lane == n ? ds : mds;
-                n += 1;
-                p = (d == ds) ? f : fmaf(ds, s, p);
-                j += cr ? u : 0;
-                const float fn = a == 0 ? xn : (float)j * dyz;
-                f = cr ? fn : f;
-                cur += (uint32_t)__builtin_amdgcn_readlane(du, ax);
-                if (ax == 0) xn = xface(j + u);
-            } while (!out && n < nmax);
-            if (!out) break;
-            /* as boundary_move */
-            const int lo = __builtin_amdgcn_readlane(neg(), ax);
-            const int bd = face_bd(cm, 2 * ax + 1 - lo);
-            if (bd == 1 || bd == 3) {
-                const bool hi_end = (bd == 1) == (lo != 0);
-                if (a == ax) {
-                    p = hi_end ? (a == 0 ? cm.Lx : (a == 1 ? cm.Ly : cm.Lz)) : 0.f;
-                    s = bd == 3 ? -s : s;
-                    is = bd == 3 ? -is : is;
-                    j = (hi_end ? nf : 1) - neg();
-                }
-            } else {
-                Ray w{};
-                w.ic = index(0); w.jc = index(1); w.kc = index(2);
-                bl = __builtin_amdgcn_readfirstlane(boundary_move<TM>(cm, sn, L, w, e, wl));
+                f = cr ? fn : fo;
+                jn += cr == eq ? 0.f : (cr ? uf : -uf);
+                cs += cr == eq ? 0 : (cr ? du : -du);
+                if (ax == 0) xn = xface((int)jn);
             }
-        }
+            fn = a == 0 ? xn : jn * dyz;
+            const unsigned long long out = __ballot(jn == past);
+            if (__builtin_expect(out != 0ull, 0)) {
+                /* as boundary_move */
+                const int ax = (int)__builtin_ctzll(out) & 3;
+                int ci = (int)jn - u + neg();
+                const int lo = __builtin_amdgcn_readlane(neg(), ax);
+                const int bd = face_bd(cm, 2 * ax + 1 - lo);
+                if (bd == 1 || bd == 3) {
+                    const bool hi_end = (bd == 1) == (lo != 0);
+                    if (a == ax) {
+                        p = hi_end ? (a == 0 ? cm.Lx : (a == 1 ? cm.Ly : cm.Lz)) : 0.f;
+                        s = bd == 3 ? -s : s;
+                        is = bd == 3 ? -is : is;
+                        ci = hi_end ? nf : 1;
+                    }
+                    enter(ci);
+                } else {
+                    Ray w{};
+                    w.ic = __builtin_amdgcn_readlane(ci, 0);
+                    w.jc = __builtin_amdgcn_readlane(ci, 1);
+                    w.kc = __builtin_amdgcn_readlane(ci, 2);
+                    bl = __builtin_amdgcn_readfirstlane(boundary_move<TM>(cm, sn, L, w, e, wl));
+                    nmax = n;
+                }
+            }
+        } while (n < nmax);
         /* the absorption terms of the n steps, one per lane (the lanes
          * from n up work on cell 0 and count for nothing) */
         float K, B;

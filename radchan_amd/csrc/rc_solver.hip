@@ -496,10 +496,10 @@ __device__ __forceinline__ void coarsen64(const DevSnap &sn, int g, int &ic, int
  *
  * 64^3, 100 rays, 2 runs (302 M steps, the longest ray 21 000): a thread per
  * cell, its wavefront waiting for the longest of 64 rays and at last for
- * the longest of all, took 2 x 17.3 ms; both runs in one launch now take 8.1
+ * the longest of all, took 2 x 17.3 ms; both runs in one launch now take 7.6
  * ms, of which 4.6 are the bulk (FP64 arithmetic, about 150 instructions per
  * step) and the rest the last rays: a lone lane's step takes about 3000
- * clocks, coop64's 430 (15.3 ms per run without it).  REFILL64 4 to 16 and
+ * clocks, coop64's 400 (15.3 ms per run without it).  REFILL64 4 to 16 and
  * STEPS64 1 to 4 are within 5 %; COOP64 4 to 16 within 1 %; 3 wavefronts per
  * SIMD instead of 4 (128 registers, a few spills) 2 % slower; stopping the
  * wavefront for a ray of over 1000 steps to march it together at once, the
@@ -534,70 +534,84 @@ __device__ int coop64(const DevCommon &cm, const DevSnap &sn, const Drain64 &r, 
     int cnt = uni64(r.cnt), g = MG ? uni64(r.g) : 0, steps = 0;
     const uint32_t row = (uint32_t)uni64((int)r.row);
     Lev64 L = lev64(sn, g);
-    /* the axis' next face j of 0..nf and its coordinate f, the unit step u,
-     * cells stride apart */
-    int j, nf, u, stride;
-    float dyz;
-    double f;
-    uint32_t c;                                         /* the cell (uniform) */
-    auto level = [&](int ic, int jc, int kc) {
-        nf = a == 0 ? L.im : (a == 1 ? L.jm : L.km);
-        stride = a == 0 ? 1 : (a == 1 ? L.im : L.im * L.jm);
-        dyz = a == 1 ? L.dy : L.dz;
-        u = s < 0.0 ? -1 : 1;
-        j = (a == 0 ? ic : (a == 1 ? jc : kc)) - (s < 0.0 ? 1 : 0);
-        c = (uint32_t)(ic - 1) + (uint32_t)L.im * ((uint32_t)(jc - 1) + (uint32_t)L.jm * (uint32_t)(kc - 1));
-    };
+    /* What a step needs first is ready before it: the face ahead, f, and the
+     * one after it, fn (index jn, as a float; past: its value once the grid
+     * is left, lane 3: none; xn: the x axis').  u: the axis' index step, cs
+     * its share of the cell index and du the share's step. */
+    double f, fn;
+    float xn, jn, past, uf, dyz;
+    int nf, u, du, cs;
+    auto neg = [&]() { return s < 0.0 ? 1 : 0; };
     auto xface = [&](int q) { return gld32(L.xu, (uint32_t)min(max(q, 0), L.im)); };
-    auto index = [&](int axis) { return __builtin_amdgcn_readlane(j + (s < 0.0 ? 1 : 0), axis); };
-    level(uni64(r.ic), uni64(r.jc), uni64(r.kc));
+    auto enter = [&](int ci) {                  /* from the axis' cell index */
+        const int j = ci - neg(), stride = a == 0 ? 1 : (a == 1 ? L.im : L.im * L.jm);
+        nf = a == 0 ? L.im : (a == 1 ? L.jm : L.km);
+        dyz = a == 1 ? L.dy : L.dz;
+        u = 1 - 2 * neg();
+        uf = (float)u;
+        du = a == 3 ? 0 : u * stride;
+        cs = a == 3 ? 0 : (ci - 1) * stride;
+        past = a == 3 ? -9.f : (neg() ? -2.f : (float)(nf + 2));
+        jn = (float)(j + u);
+        f = a == 0 ? (double)xface(j) : (a == 3 ? 1e300 : (double)((float)j * dyz));
+        xn = xface(j + u);
+        fn = (double)(a == 0 ? xn : jn * dyz);
+    };
+    auto cell = [&]() { return (int)jn - u + neg(); };
+    enter(a == 0 ? r.ic : (a == 1 ? r.jc : r.kc));
     for (;;) {
         int n = 0, end = -1;
         double pds = 0.0;
         uint32_t pc = 0;
-        const int cap = min(64, L.maxs - cnt);
-        while (n < cap && end < 0) {
-            /* (re)entered after a boundary */
-            const int last = s < 0.0 ? 0 : nf, du = u * stride;
-            float xn = xface(j + u);                    /* the x face after the next */
-            f = a == 0 ? (double)xface(j) : (a == 3 ? 1e300 : (double)((float)j * dyz));
-            int ax;
-            bool ev;
-            do {
-                const double d = (f - p) * is;
-                double m = d, o = quad64<0xB1>(d);
-                m = o < m ? o : m;
-                o = quad64<0x4E>(m);
-                m = o < m ? o : m;
-                /* the tie rules: z before y before x (and z if nothing compares) */
-                ax = (0xAA52 >> (2 * (int)(__ballot(d == m) & 7ull))) & 3;
+        int nmax = min(64, L.maxs - cnt);
+        do {
+            const double d = (f - p) * is;
+            double m = d, o = quad64<0xB1>(d);
+            m = o < m ? o : m;
+            o = quad64<0x4E>(m);
+            m = o < m ? o : m;
+            const bool eq = d == m;
+            const int ea = (int)__ballot(eq) & 7;
+            const double fo = f, pm = fma(m, s, p);
+            f = eq ? fn : f;
+            p = eq ? fo : pm;
+            const int cq = cs + quad_lane<0xB1>(cs);
+            const int c = cq + quad_lane<0x4E>(cq);
+            if (lane == n) { pds = m; pc = (uint32_t)c; }
+            ++n;
+            jn += eq ? uf : 0.f;
+            cs += eq ? du : 0;
+            if (__builtin_expect(((0x14 >> ea) & 1) == 0, 0)) {
+                /* x crossed, or faces of several axes at once: the tie
+                 * rules, z before y before x (z if nothing compares) */
+                const int ax = (0xAA52 >> (2 * ea)) & 3;
                 const bool cr = a == ax;
-                ev = (__ballot(j == last) & (7ull & (1ull << ax))) != 0ull;
-                if (lane == n) { pds = m; pc = c; }
-                ++n;
-                p = (d == m) ? f : fma(m, s, p);
-                j += cr ? u : 0;
-                const double fn = a == 0 ? (double)xn : (double)((float)j * dyz);
-                f = cr ? fn : f;
-                c += (uint32_t)__builtin_amdgcn_readlane(du, ax);
-                if (ax == 0) xn = xface(j + u);
-            } while (!ev && n < cap);
-            if (!ev) break;
-            const int d = __builtin_amdgcn_readlane(s < 0.0 ? 1 : 0, ax), face = 2 * ax + 1 - d;
-            const int bd = (int)(bds >> (4 * face)) & 15;
-            if (bd == 1 || bd == 3) {                             /* periodic, specular: on from one of the sides */
-                const bool hi = (d != 0) == (bd == 1);
-                if (a == ax) {
-                    p = hi ? (double)(a == 0 ? cm.Lx : (a == 1 ? cm.Ly : cm.Lz)) : 0.0;
-                    if (bd == 3) { s = -s; is = -is; u = s < 0.0 ? -1 : 1; }
-                    j = (hi ? nf : 1) - (s < 0.0 ? 1 : 0);
-                }
-                const int ic = index(0), jc = index(1), kc = index(2);
-                c = (uint32_t)(ic - 1) + (uint32_t)L.im * ((uint32_t)(jc - 1) + (uint32_t)L.jm * (uint32_t)(kc - 1));
-            } else {
-                end = face;
+                f = cr ? fn : fo;
+                jn += cr == eq ? 0.f : (cr ? uf : -uf);
+                cs += cr == eq ? 0 : (cr ? du : -du);
+                if (ax == 0) xn = xface((int)jn);
             }
-        }
+            fn = (double)(a == 0 ? xn : jn * dyz);
+            const unsigned long long out = __ballot(jn == past);
+            if (__builtin_expect(out != 0ull, 0)) {
+                const int ax = (int)__builtin_ctzll(out) & 3, lo = __builtin_amdgcn_readlane(neg(), ax);
+                const int face = 2 * ax + 1 - lo, bd = (int)(bds >> (4 * face)) & 15;
+                if (bd == 1 || bd == 3) {                         /* periodic, specular: on from one of the sides */
+                    const bool hi = (lo != 0) == (bd == 1);
+                    int ci = cell();
+                    if (a == ax) {
+                        p = hi ? (double)(a == 0 ? cm.Lx : (a == 1 ? cm.Ly : cm.Lz)) : 0.0;
+                        s = bd == 3 ? -s : s;
+                        is = bd == 3 ? -is : is;
+                        ci = hi ? nf : 1;
+                    }
+                    enter(ci);
+                } else {
+                    end = face;
+                    nmax = n;
+                }
+            }
+        } while (n < nmax);
         /* attenuation of the block's steps (:358-370) */
         double em = 0.0, ex = 1.0, fac = 0.0;
         if (lane < n) {
@@ -643,19 +657,23 @@ __device__ int coop64(const DevCommon &cm, const DevSnap &sn, const Drain64 &r, 
         steps += m;
         cnt += m;
         if (m == n && end >= 0) {
-            const Ray rr{index(0), index(1), index(2), 0, 0, 0};
+            const int ci = cell();
+            const Ray rr{__builtin_amdgcn_readlane(ci, 0), __builtin_amdgcn_readlane(ci, 1), __builtin_amdgcn_readlane(ci, 2),
+                         0, 0, 0};
             de -= wall64(cm, sn, L, row, end, rr, W, tra, Bi, rBi);
             break;
         }
         if (stop) break;
         if (cnt >= L.maxs) {
             if (!MG || g >= cm.grid_num - 1) break;
-            int ic = index(0), jc = index(1), kc = index(2);
+            const int ci = cell();
+            int ic = __builtin_amdgcn_readlane(ci, 0), jc = __builtin_amdgcn_readlane(ci, 1),
+                kc = __builtin_amdgcn_readlane(ci, 2);
             coarsen64(sn, g, ic, jc, kc);
             g += 1;
             cnt = 0;
             L = lev64(sn, g);
-            level(ic, jc, kc);
+            enter(a == 0 ? ic : (a == 1 ? jc : kc));
         }
     }
     de_out = de;
