@@ -44,12 +44,6 @@ using namespace rcd;
 
 namespace rc {
 
-/* the median of x, y, z (v_med3_u32): with z all ones the larger of x and
- * y, with z 0 the smaller */
-__device__ __forceinline__ uint32_t umed3(uint32_t x, uint32_t y, uint32_t z) {
-    return max(min(x, y), min(max(x, y), z));
-}
-
 /* bitonic sort of 64 R keys held in registers, element R lane + r in x[r]:
  * compare-exchanges at distances below R stay inside a lane; the stages at
  * distance R..32 R exchange with lane (lane ^ distance/R) (21 of them).  No

@@ -28,17 +28,21 @@
  *   (4) per occupied bin, ff summed in ascending h by one thread from the
  *       pair weights staged in LDS -- the reference's order, so ff is bit
  *       for bit the reference's;
- *   (5) the gg chain (one lane, descending bins) and the k_avg sum (one lane
- *       of another wave, ascending bins): the reference's sequences of
+ *   (5) the gg chain (a row of lanes, descending bins) and the k_avg sum (the
+ *       next row, ascending bins): the reference's sequences of
  *       operations with the zero terms of empty bins left out (x - 0 and
  *       x + 0 are exact), so both are bit for bit given the same kk;
  *   (6) one thread per quadrature point: binary searches for the first
  *       occupied bin whose gg reaches gq[r].
- * The bin index uses the device's FP64 pow, which may differ from the host
- * libm's in the last bit, and kk = (h step + pmin)^(1/pwr) is formed by
+ * The bin index is the one of the device's FP64 pow, which may differ from
+ * the host libm's in the last bit, and kk = (h step + pmin)^(1/pwr) is formed by
  * squaring when 1/pwr is an integer (10 for pwr = 0.1), within 5 ulp of
  * pow: results agree with the CPU restatement to FP64 rounding (and a pair
  * exactly on a bin edge could land one bin over).
+ *
+ * 47 580 spectra of 1000 points (770 MB): 1.48 -> 0.90 ms.  The bound was the
+ * sums' LDS accesses (0.65 ms), then FP64 pow and the sort's instructions; now
+ * what is left of the sums (about 0.3 ms), the sort and LDS latencies.
  *
  * LDS per spectrum, np2 = 256 R >= n - 1 (R = 1, 2, .., 32 keys per thread,
  * one kernel instance each, chosen by the launch's longest spectrum): keys u32[np2], run
@@ -52,6 +56,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "rc_device.h"
@@ -85,39 +90,39 @@ __device__ __forceinline__ void block_sort(uint32_t (&x)[R], uint32_t *K, int ti
     int base = tid * R;
     /* opaque, so the per-stage masks are formed here rather than hoisted */
     asm volatile("" : "+v"(base));
+    /* bit b of v as all ones or 0 */
+    auto bit = [](int v, int b) { return (uint32_t)((v << (31 - b)) >> 31); };
 #pragma unroll
-    for (int k = 2; k <= 256 * R; k <<= 1) {
+    for (int kb = 1; (1 << kb) <= 256 * R; ++kb) {
+        const int k = 1 << kb;
 #pragma unroll
-        for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int jb = kb - 1; jb >= 0; --jb) {
+            const int j = 1 << jb;
             if (j < R) {
+                /* descending where bit kb is set */
+                const uint32_t down = k < R || k >= 256 * R ? 0u : bit(base, kb);
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const int p = r ^ j;
                     if (p > r) {
-                        const bool up = ((base + r) & k) == 0;
-                        const uint32_t lo = min(x[r], x[p]), hi = max(x[r], x[p]);
-                        x[r] = up ? lo : hi;
-                        x[p] = up ? hi : lo;
+                        const uint32_t d = k < R ? ((r & k) ? ~0u : 0u) : down, u = x[r], w = x[p];
+                        x[r] = umed3(u, w, d);
+                        x[p] = umed3(u, w, ~d);
                     }
                 }
-            } else if (j < 64 * R) {
-                const bool keep_min = ((base & j) == 0) == ((base & k) == 0);
+                continue;
+            }
+            const uint32_t keep_max = bit(k >= 256 * R ? base : base ^ (base >> (kb - jb)), jb);
+            if (j < 64 * R) {
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const uint32_t y = lane_xor(x[r], j / R);
-                    x[r] = keep_min ? min(x[r], y) : max(x[r], y);
-                }
+                for (int r = 0; r < R; ++r) x[r] = umed3(x[r], lane_xor(x[r], j / R), keep_max);
             } else {
                 __syncthreads();
 #pragma unroll
                 for (int r = 0; r < R; ++r) K[base + r] = x[r];
                 __syncthreads();
-                const bool keep_min = ((base & j) == 0) == ((base & k) == 0);
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const uint32_t y = K[(base + r) ^ j];
-                    x[r] = keep_min ? min(x[r], y) : max(x[r], y);
-                }
+                for (int r = 0; r < R; ++r) x[r] = umed3(x[r], K[(base + r) ^ j], keep_max);
             }
         }
     }
@@ -131,6 +136,10 @@ __device__ __forceinline__ void block_sort(uint32_t (&x)[R], uint32_t *K, int ti
  * generator's pwr = 0.1: four products, within 5 ulp of the rounded power),
  * else pow */
 __device__ __forceinline__ double kpow(double x, double ipwr, int ie) {
+    if (ie == 10) {                     /* (the loop's products) */
+        const double x2 = x * x, x4 = x2 * x2;
+        return x2 * (x4 * x4);
+    }
     if (ie > 0) {
         double r = 1.0, b = x;
         for (int e = ie; e; e >>= 1) {
@@ -156,6 +165,85 @@ __device__ __noinline__ double kk_at_q(int h, double step, double pmin, double i
     return kk_at(h, step, pmin, ipwr, ie);
 }
 
+/* 2^y: y = n + f, the Taylor series of exp(f ln 2) to the 13th power, |f| <= 1/2 */
+__device__ __forceinline__ double exp2_d(double y) {
+    const double n = rint(y), r = (y - n) * 0.6931471805599453;
+    double p = 1.0 / 6227020800.0;
+    p = fma(r, p, 1.0 / 479001600.0);
+    p = fma(r, p, 1.0 / 39916800.0);
+    p = fma(r, p, 1.0 / 3628800.0);
+    p = fma(r, p, 1.0 / 362880.0);
+    p = fma(r, p, 1.0 / 40320.0);
+    p = fma(r, p, 1.0 / 5040.0);
+    p = fma(r, p, 1.0 / 720.0);
+    p = fma(r, p, 1.0 / 120.0);
+    p = fma(r, p, 1.0 / 24.0);
+    p = fma(r, p, 1.0 / 6.0);
+    p = fma(r, p, 0.5);
+    p = fma(r, p, 1.0);
+    p = fma(r, p, 1.0);
+    return __builtin_amdgcn_ldexp(p, (int)n);
+}
+/* k^pwr to about 1e-14 |pwr|, k a normal float: log2 k in FP32, l, corrected by
+ * the logarithm of k 2^-l = 1 + d, |d| < 1e-5 */
+__device__ __forceinline__ double pow_near(double k, double pwr) {
+    const double l = (double)__builtin_amdgcn_logf((float)k);
+    const double d = fma(k, exp2_d(-l), -1.0);
+    const double c = d * fma(d, fma(d, 1.0 / 3.0, -0.5), 1.0) * 1.4426950408889634;
+    return exp2_d(pwr * (l + c));
+}
+
+/* the bin of a pair, as the reference forms it; out of line, since few pairs
+ * need it */
+__device__ __noinline__ int pair_bin(double ki, double pwr, double pmin, double step, int n_pwrk) {
+    const double xb = (pow(ki, pwr) - pmin) / step + 1;
+    return min(max(0, (int)xb), n_pwrk);
+}
+
+/* lane K of the row's x, in every lane of the row (a DPP row_newbcast) */
+template <int K>
+__device__ __forceinline__ double row_lane(double x) {
+    return __builtin_amdgcn_update_dpp(0.0, x, 0x150 + K, 0xF, 0xF, true);
+}
+template <int... K>
+__device__ __forceinline__ double ordered_16(double v, const double (&m)[16], double acc, std::integer_sequence<int, K...>) {
+    ((acc = fma(row_lane<K>(v), m[K], acc)), ...);
+    return acc;
+}
+
+/* The sums acc + sg p[0], acc + sg p[0] + sg p[-1], .. (n of them, each
+ * addition rounded, in that order) in place of p[0], p[-1], ..; returns the
+ * last.  By a row of 16 lanes, l the lane's place in it: 16 values are read
+ * at once, and each is broadcast and added in every lane that comes after
+ * it, or added 0 times before it, so that lane l is left with the l-th sum.
+ * With a lane reading and writing one value at a time the LDS accesses,
+ * which take as long for one lane as for 64, were the bound: 0.65 of the
+ * kernel's 1.34 ms at 47 580 spectra of 1000 points. */
+__device__ __forceinline__ double ordered_sums(double *p, int n, int l, double sg, double acc) {
+    double m[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) m[k] = k <= l ? sg : 0.0;
+    p -= l;
+    double v = l < n ? *p : 0.0;
+    for (; n > 0; n -= 16, p -= 16) {
+        const double nv = l < n - 16 ? p[-16] : 0.0;
+        if (__ballot(!(fabs(v) < 1e300)) == 0ull) {
+            acc = ordered_16(v, m, acc, std::make_integer_sequence<int, 16>{});
+        } else {
+            /* 0 times infinity is not 0 */
+            const double w = v;
+            for (int k = 0; k < 16; ++k) {
+                const double b = __shfl(w, k, 16);
+                acc = k <= l ? acc + sg * b : acc;
+            }
+        }
+        if (l < n) *p = acc;
+        acc = row_lane<15>(acc);
+        v = nv;
+    }
+    return acc;
+}
+
 /* gg(j) = G_lo of the first occupied bin above j, 1 above the last */
 __device__ __forceinline__ double gg_at(int j, const uint16_t *RB, const double *G, int r0, int r1) {
     int lo = r0, hi = r1;
@@ -166,8 +254,10 @@ __device__ __forceinline__ double gg_at(int j, const uint16_t *RB, const double 
     return lo < r1 ? G[lo] : 1.0;
 }
 
+/* up to 1024 pairs: 7 workgroups per CU (72 registers, a few spilled), 1.03 ms at 47 580 spectra of 1000 points; unbounded (82
+ * registers, 5 workgroups) 1.19, 6 1.06, 8 (64 registers) 1.11 */
 template <int R>
-__global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
+__global__ __launch_bounds__(CK_THREADS, R <= 4 ? 7 : 1) void k_ckdist(CkArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ double red_lo[CK_WAVES], red_hi[CK_WAVES];
     __shared__ int scan[CK_WAVES];
@@ -176,11 +266,11 @@ __global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
     const int s = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     constexpr int np2 = CK_THREADS * R;
-    uint32_t *K = (uint32_t *)lds;                      /* [np2] sort keys          */
+    uint16_t *RB = (uint16_t *)lds;                     /* [np2] run bins           */
+    uint32_t *K = (uint32_t *)(lds + 2 * (size_t)np2);  /* [np2] sort keys          */
     uint32_t *RS = K + np2;                             /* [np2] run starts         */
-    double *P = (double *)lds;                          /* [np2] kk*ff (over K, RS) */
-    double *F = (double *)(lds + 8 * (size_t)np2);      /* [np2] ff, then gg below  */
-    uint16_t *RB = (uint16_t *)(lds + 16 * (size_t)np2); /* [np2] run bins          */
+    double *P = (double *)K;                            /* [np2] kk*ff from the last bin (over K, RS) */
+    double *F = P + np2;                                /* [np2] ff, then gg below  */
 
     const int64_t base = a.off[s];
     const int64_t n64 = a.off[s + 1] - base;
@@ -223,7 +313,19 @@ __global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
     const int npair = n > 1 ? n - 1 : 0;
 
     /* (2) keys: bin << 13 | h for the pair (h-1, h), pair i = R tid + r in
-     * x[r]; padding sorts last */
+     * x[r]; padding sorts last.  Where 1/pwr is an integer e, ki^pwr is the
+     * FP32 power (within 1e-6 for e = 10) and one Newton step on p^e = ki in
+     * FP64, which leaves (e - 1)/2 (1e-6)^2, else pow_near; the bin is taken
+     * from it unless it lies so close to an edge (`near`, 10 times that or
+     * more, and rounding) that the power's rounding could matter.  About 20
+     * (60) instructions for pow's 170: 16 000 spectra of 1000 points, pwr
+     * 0.1 (0.15), 0.56 -> 0.34 ms (0.67 -> 0.59) with the sums below.
+     * The weights' quotients by the band's width: RN(1/width) and two
+     * residual corrections by fma, the rounded quotient (Markstein 1990). */
+    const double rstep = 1.0 / step, rw = 1.0 / width, re = a.pwr;
+    const float pwrf = (float)a.pwr;
+    const double near = pmax * rstep * (a.ie > 0 ? 5e-12 * max(a.ie, 6) : 1e-12 * fmax(a.pwr, 1.0)) + 1e-9;
+    const bool wide = width >= 1e-100 && width <= 1e100;
     uint32_t x[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -234,12 +336,29 @@ __global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
             const double ki = (kvs[h] + kvs[h - 1]) / 2;
             int bin = 1;                                 /* a flat spectrum (step 0) */
             if (step > 0.0) {
-                const double xb = (pow(ki, a.pwr) - pmin) / step + 1;
-                bin = max(0, (int)xb);
-                bin = min(bin, n_pwrk);
+                double pk;
+                if (a.ie > 0) {
+                    const float kf = (float)ki;
+                    const double p0 = (double)__builtin_amdgcn_exp2f(pwrf * __builtin_amdgcn_logf(kf));
+                    const double c = (kpow(p0, a.ipwr, a.ie) - ki) * (double)__builtin_amdgcn_rcpf(kf);
+                    pk = fma(-p0 * c, re, p0);
+                } else {
+                    pk = pow_near(ki, a.pwr);
+                }
+                const double xb = (pk - pmin) * rstep + 1;
+                const double fr = xb - floor(xb);
+                bin = min((int)xb, n_pwrk);
+                if (!(fr > near && fr < 1.0 - near && xb >= 1.0 && ki >= 1e-30 && ki <= 1e30))
+                    bin = pair_bin(ki, a.pwr, pmin, step, n_pwrk);
             }
             key = ((uint32_t)bin << CK_IDX_BITS) | (uint32_t)h;
-            F[i] = (wvs[h] - wvs[h - 1]) / width;        /* the pair's weight, by pair */
+            /* the pair's weight, by pair */
+            const double dw = wvs[h] - wvs[h - 1];
+            double w = dw * rw;
+            w = fma(fma(-w, width, dw), rw, w);
+            w = fma(fma(-w, width, dw), rw, w);
+            if (!(wide && fabs(dw) >= 1e-100 && fabs(dw) <= 1e100)) w = dw / width;
+            F[i] = w;
         }
         x[r] = key;
     }
@@ -297,7 +416,7 @@ __global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
     /* kk*ff of the bins the k_avg sum covers (1..ng), over the dead keys */
     for (int r = tid; r < m; r += CK_THREADS) {
         const int bin = RB[r];
-        P[r] = (bin >= 1 && bin <= ng) ? kk_at(bin, step, pmin, a.ipwr, a.ie) * F[r] : 0.0;
+        P[m - 1 - r] = (bin >= 1 && bin <= ng) ? kk_at(bin, step, pmin, a.ipwr, a.ie) * F[r] : 0.0;
     }
     if (tid == 0) {
         int r0 = (m > 0 && RB[0] == 0) ? 1 : 0;
@@ -308,32 +427,19 @@ __global__ __launch_bounds__(CK_THREADS) void k_ckdist(CkArgs a) {
     __syncthreads();
     const int r0 = s_r0, r1 = s_r1;
 
-    /* (5) gg chain from the top (wave 0) and the k_avg sum (wave 1) */
-    if (tid == 0) {
-        double g = 1.0;
-        int r = r1 - 1;
-        for (; r - 7 >= r0; r -= 8) {
-            double f[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) f[u] = F[r - u];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) { g = g - f[u]; F[r - u] = g; }
+    /* (5) the gg chain from the top bin down, and the k_avg sum from the
+     * bottom bin up (P is the other way round), by the first two rows of a
+     * wavefront (ordered_sums).  The wavefront goes round with the workgroup:
+     * the same one in every workgroup would be one SIMD's work. */
+    if (wv == (int)(blockIdx.x & (CK_WAVES - 1)) && lane < 32) {
+        const bool avg = lane >= 16;
+        const double acc = ordered_sums(avg ? P + (m - 1 - r0) : F + (r1 - 1), r1 - r0, lane & 15, avg ? 1.0 : -1.0,
+                                        avg ? 0.0 : 1.0);
+        if (lane == 16) {
+            a.kavg[s] = acc;
+            a.kmin[s] = lo;
+            a.kmax[s] = hi;
         }
-        for (; r >= r0; --r) { g = g - F[r]; F[r] = g; }
-    } else if (tid == 64) {
-        double acc = 0.0;
-        int r = r0;
-        for (; r + 7 < r1; r += 8) {
-            double v[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = P[r + u];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) acc = acc + v[u];
-        }
-        for (; r < r1; ++r) acc = acc + P[r];
-        a.kavg[s] = acc;
-        a.kmin[s] = lo;
-        a.kmax[s] = hi;
     }
     __syncthreads();
 

@@ -66,6 +66,12 @@ __device__ __forceinline__ uint32_t lane_xor(uint32_t v, int m) {
     }
 }
 
+/* the median of x, y, z (v_med3_u32): with z all ones the larger of x and
+ * y, with z 0 the smaller */
+__device__ __forceinline__ uint32_t umed3(uint32_t x, uint32_t y, uint32_t z) {
+    return max(min(x, y), min(max(x, y), z));
+}
+
 /* ---- Philox4x32-10 (Salmon, Moraes, Dror, Shaw, "Parallel random numbers:
  * as easy as 1, 2, 3", SC'11): 10 rounds of two 32x32->64 multiplies with
  * a Weyl-sequence key schedule. ---------------------------------------- */
