@@ -173,13 +173,10 @@ size_t batched_srt_keys(const DevCommon &cm, long nunit_cells, int wg_per_cu);
 void launch_zero(hipStream_t st, double *p, size_t n);
 /* The solve's counters (rays, steps, capped, bulk slots, bulk steps) in
  * STAT_LINES copies 256 bytes apart, a workgroup adding to the copy of its
- * index: every wavefront adds its own, and one line takes about 90 adds per
+ * index (stat_line): every wavefront adds its own, and one line takes about 90 adds per
  * microsecond (8192 wavefronts on one line: 0.37 ms of a 16^3 solve).  The
  * host sums them. */
 constexpr int STAT_LINES = 32, STAT_STRIDE = 32, STAT_WORDS = STAT_LINES * STAT_STRIDE;
-__device__ inline unsigned long long *stat_line(unsigned long long *stats) {
-    return stats + (blockIdx.x % STAT_LINES) * STAT_STRIDE;
-}
 void launch_zero_u64(hipStream_t st, unsigned long long *p, int n);
 /* k and Ib of every table row at each snapshot's Tmax, to its kbm, and the
  * quarter entries of its g CDFs, to its cdf_g4 */

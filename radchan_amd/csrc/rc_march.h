@@ -16,6 +16,11 @@
 
 namespace rc {
 
+/* the workgroup's copy of the solve's counters */
+__device__ inline unsigned long long *stat_line(unsigned long long *stats) {
+    return stats + (blockIdx.x % STAT_LINES) * STAT_STRIDE;
+}
+
 using namespace rcd;
 
 /* ------------------------------------------------------------------------ */
