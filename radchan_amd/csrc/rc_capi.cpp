@@ -192,7 +192,9 @@ int build_tableset(rc_ctx *c, const Tables &t, TableSet &ts, std::vector<int32_t
     for (int r = 0; r < nB; ++r) {
         const int b = idx[r];
         for (int q = 0; q < nT; ++q)
-            brow[q] = gt ? (float)(kStefan * std::pow((double)t.Tnb[q], 4) / kPi) : planck(t.Tnb[q], t.wvc[b]);
+            brow[q] = gt              ? (float)(kStefan * std::pow((double)t.Tnb[q], 4) / kPi)
+                      : t.ib.size() ? t.ib[(size_t)q * nB + b]
+                                    : planck(t.Tnb[q], t.wvc[b]);
         brow[nT] = brow[nT - 1];
         for (int g = 0; g < nQ; ++g) {
             float2 *row = &kb[((size_t)r * nQ + g) * S];

@@ -28,6 +28,9 @@ const char *last_error();
 struct Tables {
     int nB = 0, nT = 0, nQ = 0;
     std::vector<float> Tnb, kP, wvl, wvr, wvc, kavg, kq, prob, probg, wq;
+    /* planck(Tnb[q], wvc[b]) at [q][b] where the tables' maker formed it
+     * (grey), else empty */
+    std::vector<float> ib;
     void resize(int nb, int nt, int nq);
     rc_tables view();
 };
