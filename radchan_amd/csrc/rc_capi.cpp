@@ -81,6 +81,43 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+/* a second stream for the walls' launch, which runs while the fluid's last
+ * rays leave most of the GPU idle (62x48x45 cells, 128 rays, two runs, two walls: the
+ * two launches 5.0 ms one after the other, 3.3 together) */
+struct WallStream {
+    hipStream_t st = nullptr;
+    hipEvent_t fork = nullptr, join = nullptr;
+    WallStream() = default;
+    WallStream(const WallStream &) = delete;
+    WallStream &operator=(const WallStream &) = delete;
+    ~WallStream() {
+        if (fork) (void)hipEventDestroy(fork);
+        if (join) (void)hipEventDestroy(join);
+        if (st) (void)hipStreamDestroy(st);
+    }
+    /* the stream, after what `main` holds; `main` itself if there is none to be had */
+    hipStream_t begin(hipStream_t main) {
+        if (!st && (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess ||
+                    hipEventCreateWithFlags(&fork, hipEventDisableTiming) != hipSuccess ||
+                    hipEventCreateWithFlags(&join, hipEventDisableTiming) != hipSuccess)) {
+            (void)hipGetLastError();
+            if (st) (void)hipStreamDestroy(st);
+            if (fork) (void)hipEventDestroy(fork);
+            st = nullptr;
+            fork = join = nullptr;
+            return main;
+        }
+        if (hipEventRecord(fork, main) != hipSuccess || hipStreamWaitEvent(st, fork, 0) != hipSuccess) return main;
+        return st;
+    }
+    /* `main` goes on after what `s` (from begin) holds */
+    hipError_t end(hipStream_t s, hipStream_t main) {
+        if (s == main) return hipSuccess;
+        const hipError_t e = hipEventRecord(join, s);
+        return e != hipSuccess ? e : hipStreamWaitEvent(main, join, 0);
+    }
+};
+
 template <class T> int upload(DevBuf &b, const std::vector<T> &v, hipStream_t st) {
     if (int e = b.ensure(v.size() * sizeof(T))) return e;
     RC_HIP(hipMemcpyAsync(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
@@ -123,6 +160,7 @@ struct rc_ctx {
     int kloc = 0, ncell = 0, nsurf = 0, zstart = 1;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evm0 = nullptr, evm1 = nullptr;
+    WallStream wall_st;
     Tables tab;
     bool have_tables = false;
     std::vector<int32_t> idx, rank_of;
@@ -854,11 +892,14 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
         }
     } else {
         DevCommon cf = cm, cw = cm;
-        cf.srt_keys = cw.srt_keys = c->srtk.as<uint16_t>();
+        cf.srt_keys = c->srtk.as<uint16_t>();
+        cw.srt_keys = cf.srt_keys + batched_srt_keys(cm, (long)nsnap * c->ncell, c->wg_per_cu);
         if (c->reduction == 1) {
             cf.ray_de = c->rayf.as<float>();
             cw.ray_de = c->rayw.as<float>();
         }
+        /* (a captured solve keeps to one stream) */
+        const hipStream_t ws = walls && timed ? c->wall_st.begin(c->stream) : c->stream;
         launch_batched(c->stream, cf, ds, nsnap, nsnap * c->ncell, 0, c->table_bf16, c->de.as<double>(),
                        c->stats.as<unsigned long long>(), c->queue.as<int>(), c->wg_per_cu, c->threshold, c->spi);
         n += 3;
@@ -867,15 +908,16 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
             ++n;
         }
         if (walls) {
-            launch_batched(c->stream, cw, ds, nsnap, nsnap * 2 * c->nsurf, 1, c->table_bf16, c->ds.as<double>(),
+            launch_batched(ws, cw, ds, nsnap, nsnap * 2 * c->nsurf, 1, c->table_bf16, c->ds.as<double>(),
                            c->stats.as<unsigned long long>(), c->queue.as<int>() + QUEUE_WORDS, c->wg_per_cu, c->threshold,
                            c->spi);
             n += 3;
             if (c->reduction == 1) {
-                launch_reduce_rays(c->stream, cw.ray_de, (size_t)nsnap * 2 * c->nsurf * p.nVar, p.photmax,
+                launch_reduce_rays(ws, cw.ray_de, (size_t)nsnap * 2 * c->nsurf * p.nVar, p.photmax,
                                    c->ds.as<double>());
                 ++n;
             }
+            RC_HIP(c->wall_st.end(ws, c->stream));
         }
     }
     if (timed) RC_HIP(hipEventRecord(c->evm1, c->stream));
@@ -937,12 +979,12 @@ int rc_run(rc_ctx *c, int variant) {
     if (variant == RC_VARIANT_PLAIN_BANDS)
         if (int e = c->bacc.ensure((size_t)c->ncell * 4)) return e;
     if (variant == RC_VARIANT_BATCHED) {
-        /* radix-sort scratch for the larger of the fluid and wall launches;
-         * a new buffer invalidates a captured graph */
+        /* radix-sort scratch of the fluid and the wall launch; a new buffer
+         * invalidates a captured graph */
         const DevCommon cm = make_common(c);
         const long ns = (long)c->snaps.size();
-        const size_t nk = std::max(batched_srt_keys(cm, ns * c->ncell, c->wg_per_cu),
-                                   p.calcwalls == 1 ? batched_srt_keys(cm, ns * 2 * c->nsurf, c->wg_per_cu) : 0);
+        const size_t nk = batched_srt_keys(cm, ns * c->ncell, c->wg_per_cu) +
+                          (p.calcwalls == 1 ? batched_srt_keys(cm, ns * 2 * c->nsurf, c->wg_per_cu) : 0);
         if (nk) {
             void *old = c->srtk.p;
             if (int e = c->srtk.ensure(nk * 2)) return e;
@@ -1293,6 +1335,7 @@ struct rc_group {
     std::vector<rc_ctx *> cs;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evm0 = nullptr, evm1 = nullptr;
+    WallStream wall_st;
     std::vector<DevSnap> h;
     DevBuf dsnap, de, ds, stats, queue, srtk;
     int wg_per_cu = 0, threshold = 0, spi = 0, refill = -1;
@@ -1405,25 +1448,29 @@ int rc_group_run(rc_group *g) {
     if (int e = g->queue.ensure(2 * QUEUE_WORDS * sizeof(int))) return e;
     DevCommon cm = make_common(c0);
     cm.refill = g->refill;
-    const size_t nk = std::max(batched_srt_keys(cm, cells, g->wg_per_cu),
-                               walls ? batched_srt_keys(cm, wcells, g->wg_per_cu) : 0);
+    const size_t nf = batched_srt_keys(cm, cells, g->wg_per_cu),
+                 nk = nf + (walls ? batched_srt_keys(cm, wcells, g->wg_per_cu) : 0);
     if (nk)
         if (int e = g->srtk.ensure(nk * 2)) return e;
     cm.srt_keys = g->srtk.as<uint16_t>();
+    DevCommon cw = cm;
+    cw.srt_keys = cm.srt_keys + nf;
     int n = 0;
     RC_HIP(hipEventRecord(g->ev0, g->stream));
     launch_zero_u64(g->stream, g->stats.as<unsigned long long>(), STAT_WORDS);
     ++n;
     RC_HIP(hipEventRecord(g->evm0, g->stream));
+    const hipStream_t ws = walls ? g->wall_st.begin(g->stream) : g->stream;
     launch_batched(g->stream, cm, g->dsnap.as<DevSnap>(), (int)g->h.size(), cells, 0, c0->table_bf16,
                    g->de.as<double>(), g->stats.as<unsigned long long>(), g->queue.as<int>(), g->wg_per_cu,
                    g->threshold, g->spi);
     n += 3;
     if (walls) {
-        launch_batched(g->stream, cm, g->dsnap.as<DevSnap>(), (int)g->h.size(), wcells, 1, c0->table_bf16,
+        launch_batched(ws, cw, g->dsnap.as<DevSnap>(), (int)g->h.size(), wcells, 1, c0->table_bf16,
                        g->ds.as<double>(), g->stats.as<unsigned long long>(), g->queue.as<int>() + QUEUE_WORDS,
                        g->wg_per_cu, g->threshold, g->spi);
         n += 3;
+        RC_HIP(g->wall_st.end(ws, g->stream));
     }
     RC_HIP(hipEventRecord(g->evm1, g->stream));
     /* each session's tallies, means and deviations into its own buffers */
