@@ -226,7 +226,8 @@ int rc_spline_restrict(const rc_params *p, int level, const float *T, float *Tc,
  * DEVICE arrays of the sizes above; asynchronous on `stream` (a
  * hipStream_t; NULL = the null stream); calls no hipMalloc/hipFree.  The
  * grid and the spline's working space live in one fixed device array of
- * RC_SPLINE_NOALLOC_FLOATS floats (64 MiB, held by every GPU the library
+ * RC_SPLINE_NOALLOC_FLOATS floats (64 MiB, and half a MiB for what depends
+ * on the grid alone, held by every GPU the library
  * runs on until the process ends); a field that needs more (about 2.7 times
  * the fine interior at level 1, e.g. 192x128x192 fits, 256x128x256 does
  * not) is refused with an error.  Calls that overlap on one GPU share that
