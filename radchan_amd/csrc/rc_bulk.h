@@ -18,9 +18,7 @@
  *    that ended since.
  *
  * Every value is the one march_core and boundary compute, so the tallies
- * are the plain march's to the bit (but for the sign of a zero, and an
- * absolute 2^-126 W in the dump after an optical depth above 87, where the
- * plain march rounds the transmissivity to 0).
+ * are the plain march's to the bit (but for the sign of a zero).
  *
  * Measured (march kernel, nVar 2, against the step that recomputed indices
  * and addresses and stepped idle lanes too): 256x128x256, 360 bands, photmax
@@ -261,25 +259,11 @@ __device__ __forceinline__ bool bulk_step(const DevCommon &cm, const S &sn, cons
         b.fx = ld_off<float>(xu, b.ix4);
     }
     if (!wall) b.pos = ld_off<float>(P, b.cell4);
-    /* absorption (phys_core_x): expm1 and exp of minus the optical depth,
-     * which a wall makes infinite and 87 bounds (expm1 -1 to the bit there;
-     * the transmissivity 2^-126 or less) */
+    /* absorption (phys_core_x), a wall's optical depth infinite */
     float K, B;
     kb_finish<TM>(b.k, K, B);
-    const float x = fmaxf(wall ? -87.0f : -(K * ds), -87.0f);
-    const float n = rintf(x * 1.44269502f);
-    float r = fmaf(-n, 0.693145752f, x);
-    r = fmaf(-n, 1.42860677e-6f, r);
-    float p = fmaf(r, (float)(1.0 / 362880.0), (float)(1.0 / 40320.0));
-    p = fmaf(r, p, (float)(1.0 / 5040.0));
-    p = fmaf(r, p, (float)(1.0 / 720.0));
-    p = fmaf(r, p, (float)(1.0 / 120.0));
-    p = fmaf(r, p, (float)(1.0 / 24.0));
-    p = fmaf(r, p, (float)(1.0 / 6.0));
-    p = fmaf(r, p, 0.5f);
-    p = fmaf(r * r, p, r);
-    const float sc = __int_as_float(((int)n + 127) << 23);
-    const float exv = fmaf(sc, p, sc), em1 = fmaf(sc, p, sc - 1.0f);
+    float em1, exv;
+    expm1_exp_step(K * ds, wall, em1, exv);
     b.fac = (B - b.Bi) * b.invBi;
     b.dacc += ((b.W * b.tra) * em1) * b.fac;
     b.tra = b.tra * exv;

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rc_expm1.h"
+
 namespace rcd {
 
 /* load through a pointer known to address global memory (pointers read from
@@ -171,56 +173,6 @@ __device__ __forceinline__ void sincos2pi(float u, float &s, float &c) {
         case 2: s = -a; c = -b; break;
         default: s = -b; c = a; break;
     }
-}
-
-/* expm1(x) and exp(x): x = n ln2 + r with |r| <= ln2/2 (Cody-Waite, fma),
- * expm1(r) from its Taylor series through r^9/9!, then rescaled by 2^n. */
-__device__ __forceinline__ void expm1_exp(float x, float &em1, float &e) {
-    const bool under = x < -87.0f;
-    float xc = under ? -87.0f : x;
-    xc = (xc > 88.0f) ? 88.0f : xc;
-    const float n = rintf(xc * 1.44269502f);
-    float r = fmaf(-n, 0.693145752f, xc);
-    r = fmaf(-n, 1.42860677e-6f, r);
-    float p = fmaf(r, (float)(1.0 / 362880.0), (float)(1.0 / 40320.0));
-    p = fmaf(r, p, (float)(1.0 / 5040.0));
-    p = fmaf(r, p, (float)(1.0 / 720.0));
-    p = fmaf(r, p, (float)(1.0 / 120.0));
-    p = fmaf(r, p, (float)(1.0 / 24.0));
-    p = fmaf(r, p, (float)(1.0 / 6.0));
-    p = fmaf(r, p, 0.5f);
-    p = fmaf(r * r, p, r);
-    const int ni = (int)n;
-    const float sc = __int_as_float((ni + 127) << 23);
-    const float ev = fmaf(sc, p, sc);
-    const float mv = (ni == 0) ? p : fmaf(sc, p, sc - 1.0f);
-    e = under ? 0.0f : ev;
-    em1 = under ? -1.0f : mv;
-}
-
-/* expm1_exp for x <= 88 (the march's exponents: minus an optical depth,
- * which is never below -0 by more than a rounding): the same values,
- * without the clamp at the top of the range */
-__device__ __forceinline__ void expm1_exp_le88(float x, float &em1, float &e) {
-    const bool under = x < -87.0f;
-    const float xc = under ? -87.0f : x;
-    const float n = rintf(xc * 1.44269502f);
-    float r = fmaf(-n, 0.693145752f, xc);
-    r = fmaf(-n, 1.42860677e-6f, r);
-    float p = fmaf(r, (float)(1.0 / 362880.0), (float)(1.0 / 40320.0));
-    p = fmaf(r, p, (float)(1.0 / 5040.0));
-    p = fmaf(r, p, (float)(1.0 / 720.0));
-    p = fmaf(r, p, (float)(1.0 / 120.0));
-    p = fmaf(r, p, (float)(1.0 / 24.0));
-    p = fmaf(r, p, (float)(1.0 / 6.0));
-    p = fmaf(r, p, 0.5f);
-    p = fmaf(r * r, p, r);
-    const int ni = (int)n;
-    const float sc = __int_as_float((ni + 127) << 23);
-    const float ev = fmaf(sc, p, sc);
-    const float mv = (ni == 0) ? p : fmaf(sc, p, sc - 1.0f);
-    e = under ? 0.0f : ev;
-    em1 = under ? -1.0f : mv;
 }
 
 /* first index with cdf[i] > R; R == 1 and past-the-end map to n-1 */

@@ -1,0 +1,78 @@
+/*
+ * rc_expm1.h -- expm1(x) and exp(x) of the FP32 march: minus an optical
+ * depth in, the absorptivity and transmissivity of a step out.
+ *
+ * Plain C++ (fmaf, rintf, a bit cast), so that the host compiles the same
+ * functions.
+ */
+#ifndef RC_EXPM1_H
+#define RC_EXPM1_H
+
+#include <math.h>
+
+#ifdef __HIP__
+#define RC_EXPM1_FN __device__ __forceinline__
+#else
+#define RC_EXPM1_FN inline
+#endif
+
+namespace rcd {
+
+/* 2^n for -127 <= n <= 127 (2^-127 as 0) */
+RC_EXPM1_FN float exp2_int(int n) {
+    const int b = (n + 127) << 23;
+    float f;
+    __builtin_memcpy(&f, &b, sizeof f);
+    return f;
+}
+
+/* x = n ln2 + r with |r| <= ln2/2 (Cody-Waite, fma); expm1(r) from its
+ * Taylor series through r^9/9! */
+RC_EXPM1_FN float expm1_reduced(float x, int &n) {
+    const float nf = rintf(x * 1.44269502f);
+    float r = fmaf(-nf, 0.693145752f, x);
+    r = fmaf(-nf, 1.42860677e-6f, r);
+    float p = fmaf(r, (float)(1.0 / 362880.0), (float)(1.0 / 40320.0));
+    p = fmaf(r, p, (float)(1.0 / 5040.0));
+    p = fmaf(r, p, (float)(1.0 / 720.0));
+    p = fmaf(r, p, (float)(1.0 / 120.0));
+    p = fmaf(r, p, (float)(1.0 / 24.0));
+    p = fmaf(r, p, (float)(1.0 / 6.0));
+    p = fmaf(r, p, 0.5f);
+    p = fmaf(r * r, p, r);
+    n = (int)nf;
+    return p;
+}
+
+/* expm1_exp for x <= 88 (the march's exponents: minus an optical depth,
+ * which is never below -0 by more than a rounding): the same values,
+ * without the clamp at the top of the range */
+RC_EXPM1_FN void expm1_exp_le88(float x, float &em1, float &e) {
+    const bool under = x < -87.0f;
+    int n;
+    const float p = expm1_reduced(under ? -87.0f : x, n);
+    const float sc = exp2_int(n);
+    const float ev = fmaf(sc, p, sc);
+    const float mv = (n == 0) ? p : fmaf(sc, p, sc - 1.0f);
+    e = under ? 0.0f : ev;
+    em1 = under ? -1.0f : mv;
+}
+
+/* expm1(x) and exp(x): expm1_reduced, rescaled by 2^n; below -87, -1 and 0 */
+RC_EXPM1_FN void expm1_exp(float x, float &em1, float &e) { expm1_exp_le88((x > 88.0f) ? 88.0f : x, em1, e); }
+
+/* expm1_exp_le88 of minus the optical depth `depth`, or of minus infinity at
+ * a wall, in the bulk march's form: beyond 87 the scale 2^-127 is a 0, which
+ * leaves exactly -1 and 0 without a select for either.  A wall or such a
+ * depth ends the ray whatever the tolerance. */
+RC_EXPM1_FN void expm1_exp_step(float depth, bool wall, float &em1, float &e) {
+    int n;
+    const float p = expm1_reduced((wall || depth > 87.0f) ? -88.0f : -depth, n);
+    const float sc = exp2_int(n);
+    e = fmaf(sc, p, sc);
+    em1 = fmaf(sc, p, sc - 1.0f);
+}
+
+}  // namespace rcd
+
+#endif
