@@ -745,6 +745,11 @@ int rc_load_tables(rc_ctx *c, const rc_tables *t) {
         if (!(c->tab.Tnb[q] > c->tab.Tnb[q - 1])) { set_error("temperature table is not increasing"); return -3; }
     if (int e = build_tableset(c, c->tab, c->nbset, c->idx, c->rank_of)) return e;
     c->have_tables = true;
+    /* what the loaded fields' rays take from the rows at Tmax */
+    if (!c->snaps.empty() && c->hsnap.size() == c->snaps.size()) {
+        launch_rows_derived(c->stream, make_common(c), c->dsnap.as<DevSnap>(), (int)c->hsnap.size());
+        RC_HIP(hipGetLastError());
+    }
     return 0;
 }
 
