@@ -23,6 +23,7 @@
 
 #include "rc_internal.h"
 #include "rc_kernels.h"
+#include "rc_scratch.h"
 
 namespace rc {
 void launch_batched(hipStream_t st, const DevCommon &cm, const DevSnap *snaps, int nsnap, int nunit_cells, int surface,
@@ -958,28 +959,17 @@ int rc_run(rc_ctx *c, int variant) {
         set_error("the per-band plain variant needs sorted band keys (srt=1, narrow band)");
         return -2;
     }
-    if (p.fp64 == 1) {
-        /* tallies of every ray of all runs, at most 2 GiB, else as many as
-         * there is memory for (one unit's at least): the launches are split
-         * to fit */
-        const size_t P = (size_t)p.photmax, nr = (size_t)std::max(c->ncell, p.calcwalls == 1 ? 2 * c->nsurf : 0) * P;
-        size_t want = std::max(std::min(nr * p.nVar, (size_t)1 << 28), P);
-        while (!c->ray64.p) {
-            if (hipMalloc(&c->ray64.p, want * 8) == hipSuccess) { c->ray64.bytes = want * 8; break; }
-            c->ray64.p = nullptr;
-            (void)hipGetLastError();
-            if (want == P) { set_error("device allocation of " + std::to_string(want * 8) + " bytes failed"); return -11; }
-            want = std::max(want / 2, P);
-        }
-        c->runs64 = (int)std::max<size_t>(1, std::min<size_t>(p.nVar, c->ray64.bytes / 8 / nr));
-    }
-    if ((variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) && p.srt == 1 && !p.grey) {
+    if (variant == RC_VARIANT_PLAIN || variant == RC_VARIANT_PLAIN_BANDS) {
+        const bool keys = p.srt == 1 && !p.grey;
         const size_t nk = (size_t)std::max(c->ncell, 2 * c->nsurf) * p.photmax;
-        if (p.fp64 == 1 && c->runs64 > 1 && c->keys.ensure(nk * c->runs64 * 2) != 0) {
-            (void)hipGetLastError();
-            c->runs64 = 1;
+        if (p.fp64 == 1) {
+            const size_t nr = (size_t)std::max(c->ncell, p.calcwalls == 1 ? 2 * c->nsurf : 0) * p.photmax;
+            c->runs64 = fp64_scratch(c->keys, c->ray64, keys ? nk : 0, nr, (size_t)p.photmax, p.nVar);
+            if (!c->runs64) return -11;
+            (void)hipGetLastError();    /* of the sizes there was no memory for */
+        } else if (keys) {
+            if (int e = c->keys.ensure(nk * 2)) return e;
         }
-        if (int e = c->keys.ensure(nk * 2)) return e;
     }
     if (variant == RC_VARIANT_PLAIN_BANDS)
         if (int e = c->bacc.ensure((size_t)c->ncell * 4)) return e;
