@@ -186,6 +186,8 @@ struct rc_ctx {
     DevBuf ray64;                           /* FP64 path: per-ray tallies of one launch */
     int runs64 = 1;                         /* and the runs they are of */
     DevBuf srtk;                            /* batched, srt above 256 keys: radix-sort scratch */
+    int srt_beside = 1;                     /* of both launches (sort_scratch)                 */
+    size_t srt_refused = 0;
     DevBuf tr_rays, tr_unit, tr_ulist, tr_out;
     rc_stats last{};
     bool launched = false;
@@ -899,13 +901,15 @@ static int enqueue_solve(rc_ctx *c, int variant, int *launches, bool timed) {
     } else {
         DevCommon cf = cm, cw = cm;
         cf.srt_keys = c->srtk.as<uint16_t>();
-        cw.srt_keys = cf.srt_keys + batched_srt_keys(cm, (long)nsnap * c->ncell, c->wg_per_cu);
+        cw.srt_keys = cf.srt_keys;
+        if (c->srt_beside) cw.srt_keys += batched_srt_keys(cm, (long)nsnap * c->ncell, c->wg_per_cu);
         if (c->reduction == 1) {
             cf.ray_de = c->rayf.as<float>();
             cw.ray_de = c->rayw.as<float>();
         }
-        /* (a captured solve keeps to one stream) */
-        const hipStream_t ws = walls && timed ? c->wall_st.begin(c->stream) : c->stream;
+        /* (a captured solve keeps to one stream, and so does one whose
+         * launches share their sort scratch) */
+        const hipStream_t ws = walls && timed && c->srt_beside ? c->wall_st.begin(c->stream) : c->stream;
         launch_batched(c->stream, cf, ds, nsnap, nsnap * c->ncell, 0, c->table_bf16, c->de.as<double>(),
                        c->stats.as<unsigned long long>(), c->queue.as<int>(), c->wg_per_cu, c->threshold, c->spi);
         n += 3;
@@ -974,17 +978,18 @@ int rc_run(rc_ctx *c, int variant) {
     if (variant == RC_VARIANT_PLAIN_BANDS)
         if (int e = c->bacc.ensure((size_t)c->ncell * 4)) return e;
     if (variant == RC_VARIANT_BATCHED) {
-        /* radix-sort scratch of the fluid and the wall launch; a new buffer
-         * invalidates a captured graph */
+        /* radix-sort scratch of the fluid and the wall launch; another
+         * buffer or layout invalidates a captured graph */
         const DevCommon cm = make_common(c);
         const long ns = (long)c->snaps.size();
-        const size_t nk = batched_srt_keys(cm, ns * c->ncell, c->wg_per_cu) +
-                          (p.calcwalls == 1 ? batched_srt_keys(cm, ns * 2 * c->nsurf, c->wg_per_cu) : 0);
-        if (nk) {
-            void *old = c->srtk.p;
-            if (int e = c->srtk.ensure(nk * 2)) return e;
-            if (c->srtk.p != old) c->drop_graph();
-        }
+        void *const old = c->srtk.p;
+        const int beside = sort_scratch(c->srtk, batched_srt_keys(cm, ns * c->ncell, c->wg_per_cu),
+                                        p.calcwalls == 1 ? batched_srt_keys(cm, ns * 2 * c->nsurf, c->wg_per_cu) : 0,
+                                        c->srt_refused);
+        if (c->srtk.p != old || beside != c->srt_beside) c->drop_graph();
+        if (beside < 0) return -11;
+        (void)hipGetLastError();        /* of a size there was no memory for */
+        c->srt_beside = beside;
     }
     if (variant == RC_VARIANT_BATCHED && c->reduction == 1) {
         const size_t ns = c->snaps.size();
@@ -1333,6 +1338,7 @@ struct rc_group {
     WallStream wall_st;
     std::vector<DevSnap> h;
     DevBuf dsnap, de, ds, stats, queue, srtk;
+    size_t srt_refused = 0;
     int wg_per_cu = 0, threshold = 0, spi = 0, refill = -1;
     rc_stats last{};
     bool launched = false;
@@ -1443,19 +1449,19 @@ int rc_group_run(rc_group *g) {
     if (int e = g->queue.ensure(2 * QUEUE_WORDS * sizeof(int))) return e;
     DevCommon cm = make_common(c0);
     cm.refill = g->refill;
-    const size_t nf = batched_srt_keys(cm, cells, g->wg_per_cu),
-                 nk = nf + (walls ? batched_srt_keys(cm, wcells, g->wg_per_cu) : 0);
-    if (nk)
-        if (int e = g->srtk.ensure(nk * 2)) return e;
+    const size_t nf = batched_srt_keys(cm, cells, g->wg_per_cu);
+    const int beside = sort_scratch(g->srtk, nf, walls ? batched_srt_keys(cm, wcells, g->wg_per_cu) : 0, g->srt_refused);
+    if (beside < 0) return -11;
+    (void)hipGetLastError();            /* of a size there was no memory for */
     cm.srt_keys = g->srtk.as<uint16_t>();
     DevCommon cw = cm;
-    cw.srt_keys = cm.srt_keys + nf;
+    if (beside) cw.srt_keys += nf;
     int n = 0;
     RC_HIP(hipEventRecord(g->ev0, g->stream));
     launch_zero_u64(g->stream, g->stats.as<unsigned long long>(), STAT_WORDS);
     ++n;
     RC_HIP(hipEventRecord(g->evm0, g->stream));
-    const hipStream_t ws = walls ? g->wall_st.begin(g->stream) : g->stream;
+    const hipStream_t ws = walls && beside ? g->wall_st.begin(g->stream) : g->stream;
     launch_batched(g->stream, cm, g->dsnap.as<DevSnap>(), (int)g->h.size(), cells, 0, c0->table_bf16,
                    g->de.as<double>(), g->stats.as<unsigned long long>(), g->queue.as<int>(), g->wg_per_cu,
                    g->threshold, g->spi);

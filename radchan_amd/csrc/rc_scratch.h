@@ -40,6 +40,22 @@ int fp64_scratch(Buf &keys, Buf &ray, size_t run_keys, size_t run_rays, size_t u
     }
 }
 
+/* The batched launches' sort scratch: 16-bit keys, `fluid` and `walls` of
+ * them.  1: both beside each other, so that the walls' launch may run while
+ * the fluid's does; 0: room for the larger, one launch after the other; < 0:
+ * neither.  refused: the size there was no memory for (0: none yet), which
+ * is not asked for again on every solve. */
+template <class Buf>
+int sort_scratch(Buf &b, size_t fluid, size_t walls, size_t &refused) {
+    const size_t both = (fluid + walls) * 2, one = std::max(fluid, walls) * 2;
+    if (both == 0 || b.bytes >= both) return 1;
+    if (!refused || both < refused) {
+        if (!b.ensure(both)) return 1;
+        if (both != one) refused = both;
+    }
+    return b.ensure(one) ? -1 : 0;
+}
+
 }  // namespace rc
 
 #endif

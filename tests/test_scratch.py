@@ -78,3 +78,39 @@ def test_fp64_keeps_to_2_GiB(tmp_path):
     const int calls = keys.calls + ray.calls;
     CHECK(rc::fp64_scratch(keys, ray, rr, rr, 100, 2) == 1 && keys.calls + ray.calls == calls);
 """)
+
+
+SORT = r"""
+    left = std::atoll(argv[3]);
+    const size_t fluid = std::atoll(argv[1]), walls = std::atoll(argv[2]);
+    const int want = std::atoi(argv[4]);
+    Buf b;
+    size_t refused = 0;
+    for (int again = 0; again < 3; ++again) {
+        const int calls = b.calls;
+        CHECK(rc::sort_scratch(b, fluid, walls, refused) == want);
+        if (want >= 0) CHECK(b.bytes >= 2 * (want ? fluid + walls : fluid > walls ? fluid : walls));
+        if (want >= 0 && again) CHECK(b.calls == calls);
+    }
+"""
+
+
+@pytest.mark.parametrize("fluid,walls,room,want", [(1000, 300, 2600, 1), (1000, 300, 2599, 0), (1000, 300, 2000, 0),
+                                                   (300, 1000, 2000, 0), (1000, 300, 1999, -1), (1000, 0, 2000, 1),
+                                                   (1000, 0, 1999, -1), (0, 0, 0, 1)])
+def test_sort_scratch(tmp_path, fluid, walls, room, want):
+    """the walls' keys beside the fluid's, else in their place"""
+    run(tmp_path, SORT, fluid, walls, room, want)
+
+
+def test_sort_scratch_grows(tmp_path):
+    """other schedules of one session: a smaller pair of sizes is tried again"""
+    run(tmp_path, r"""
+    left = 2000;
+    Buf b;
+    size_t refused = 0;
+    CHECK(rc::sort_scratch(b, 900, 300, refused) == 0 && refused == 2400);
+    CHECK(rc::sort_scratch(b, 600, 200, refused) == 1);
+    CHECK(rc::sort_scratch(b, 700, 250, refused) == 1 && b.bytes == 1900);
+    CHECK(rc::sort_scratch(b, 900, 300, refused) == 0 && b.bytes == 1900);
+""")
