@@ -267,9 +267,12 @@ __device__ __forceinline__ bool bulk_step(const DevCommon &cm, const S &sn, cons
     b.fac = (B - b.Bi) * b.invBi;
     b.dacc += ((b.W * b.tra) * em1) * b.fac;
     b.tra = b.tra * exv;
-    if (open && b.kt == KT_LOST && !(b.tra < tol)) {      /* lost: ends without a dump */
-        b.tra = 0.f;
-        b.fac = 0.f;
+    if (__builtin_expect(open, 0)) {
+        asm volatile("");       /* a branch: as selects in every step, 2 % of a BF16 ensemble */
+        if (b.kt == KT_LOST && !(b.tra < tol)) {      /* lost: ends without a dump */
+            b.tra = 0.f;
+            b.fac = 0.f;
+        }
     }
     return !(b.tra > tol);
 }

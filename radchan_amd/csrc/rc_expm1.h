@@ -64,10 +64,14 @@ RC_EXPM1_FN void expm1_exp(float x, float &em1, float &e) { expm1_exp_le88((x > 
 /* expm1_exp_le88 of minus the optical depth `depth`, or of minus infinity at
  * a wall, in the bulk march's form: beyond 87 the scale 2^-127 is a 0, which
  * leaves exactly -1 and 0 without a select for either.  A wall or such a
- * depth ends the ray whatever the tolerance. */
+ * depth ends the ray whatever the tolerance.  (The wall's depth selected
+ * first: with one select on either condition, whose masks meet in a scalar
+ * instruction, the march of 64^3 took 7.5 ms instead of 7.3, that of
+ * 192x128x192 at three levels 49.7 instead of 49.1.) */
 RC_EXPM1_FN void expm1_exp_step(float depth, bool wall, float &em1, float &e) {
     int n;
-    const float p = expm1_reduced((wall || depth > 87.0f) ? -88.0f : -depth, n);
+    const float d = wall ? INFINITY : depth;
+    const float p = expm1_reduced(d > 87.0f ? -88.0f : -d, n);
     const float sc = exp2_int(n);
     e = fmaf(sc, p, sc);
     em1 = fmaf(sc, p, sc - 1.0f);
