@@ -59,6 +59,7 @@
 #include <utility>
 #include <vector>
 
+#include "rc_ckbin.h"
 #include "rc_device.h"
 #include "rc_internal.h"
 
@@ -76,9 +77,17 @@ struct CkArgs {
     const int64_t *off;
     const double *wvn, *kvn, *wvl, *wvr, *gq;
     double *kq, *kavg, *kmin, *kmax;
-    double pwr, ipwr;
+    double pwr, ipwr, edge;
     int nq, n_pwrk, ie;
 };
+/* the bin law's exponent: 1/pwr, that as an integer up to 64 if it is one
+ * (else 0), and the margin around a bin's edges (ck_edge_margin) */
+void ck_law(CkArgs &a, double pwr) {
+    a.pwr = pwr;
+    a.ipwr = 1.0 / pwr;
+    a.ie = (a.ipwr == std::rint(a.ipwr) && a.ipwr >= 1.0 && a.ipwr <= 64.0) ? (int)a.ipwr : 0;
+    a.edge = ck_edge_margin(a.ie, pwr);
+}
 
 /* bitonic sort of 256 R keys held in registers, element R tid + r in x[r]:
  * stages at distance below R stay inside a thread, distances R..32 R
@@ -314,17 +323,16 @@ __global__ __launch_bounds__(CK_THREADS, R <= 4 ? 7 : 1) void k_ckdist(CkArgs a)
 
     /* (2) keys: bin << 13 | h for the pair (h-1, h), pair i = R tid + r in
      * x[r]; padding sorts last.  Where 1/pwr is an integer e, ki^pwr is the
-     * FP32 power (within 1e-6 for e = 10) and one Newton step on p^e = ki in
-     * FP64, which leaves (e - 1)/2 (1e-6)^2, else pow_near; the bin is taken
-     * from it unless it lies so close to an edge (`near`, 10 times that or
-     * more, and rounding) that the power's rounding could matter.  About 20
+     * FP32 power and one Newton step on p^e = ki in FP64, else pow_near; the
+     * bin is taken from it unless it lies so close to an edge (`near`:
+     * ck_edge_margin, and rounding) that the power's error could matter.  About 20
      * (60) instructions for pow's 170: 16 000 spectra of 1000 points, pwr
      * 0.1 (0.15), 0.56 -> 0.34 ms (0.67 -> 0.59) with the sums below.
      * The weights' quotients by the band's width: RN(1/width) and two
      * residual corrections by fma, the rounded quotient (Markstein 1990). */
     const double rstep = 1.0 / step, rw = 1.0 / width, re = a.pwr;
     const float pwrf = (float)a.pwr;
-    const double near = pmax * rstep * (a.ie > 0 ? 5e-12 * max(a.ie, 6) : 1e-12 * fmax(a.pwr, 1.0)) + 1e-9;
+    const double near = pmax * rstep * a.edge + 1e-9;
     const bool wide = width >= 1e-100 && width <= 1e100;
     uint32_t x[R];
 #pragma unroll
@@ -546,9 +554,7 @@ extern "C" int rc_ckdist_device(int nspec, const int64_t *off, const double *wvn
     CkArgs a;
     a.off = off; a.wvn = wvn; a.kvn = kvn; a.wvl = wvl; a.wvr = wvr; a.gq = gq;
     a.kq = kq; a.kavg = kavg; a.kmin = kmin; a.kmax = kmax;
-    a.pwr = pwr;
-    a.ipwr = 1.0 / pwr;
-    a.ie = (a.ipwr == std::rint(a.ipwr) && a.ipwr >= 1.0 && a.ipwr <= 64.0) ? (int)a.ipwr : 0;
+    ck_law(a, pwr);
     a.nq = nq;
     a.n_pwrk = n_pwrk;
     const hipError_t e = ck_launch(a, nspec, np2, (hipStream_t)stream);
@@ -638,9 +644,7 @@ extern "C" int rc_ckdist(int nspec, const int64_t *off, const double *wvn, const
         a.kavg = (double *)d_kavg.p;
         a.kmin = (double *)d_kmin.p;
         a.kmax = (double *)d_kmax.p;
-        a.pwr = pwr;
-        a.ipwr = 1.0 / pwr;
-        a.ie = (a.ipwr == std::rint(a.ipwr) && a.ipwr >= 1.0 && a.ipwr <= 64.0) ? (int)a.ipwr : 0;
+        ck_law(a, pwr);
         a.nq = nq;
         a.n_pwrk = n_pwrk;
         CK_TRY(hipEventRecord(e0, st));
