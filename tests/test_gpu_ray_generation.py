@@ -74,3 +74,47 @@ def test_guide_edges(steps):
     tab.prob[:] = np.ceil(tab.prob * steps) / steps
     p = P.base_params(4, 4, 4, photmax=200, nVar=2, fact_mesh=1.5, seed=steps)
     solve_both(p, tab, F.channel_field(p, 600.0, 1500.0, noise=0.02, seed=2))
+
+
+@pytest.mark.parametrize("photmax", [100, 300])
+@pytest.mark.parametrize("a,b", [(2, 3), (3, 4), (7, 8), (10, 12)])
+def test_row_that_decreases(photmax, a, b):
+    """g CDF rows of 16 with two entries exchanged: the count of entries up
+    to R does not see their order, so the draws are those of the sorted rows;
+    a search by quarters would find others"""
+    tab = synthetic_nb()
+    mixed = tab.copy()
+    mixed.probg[:, ::5, a], mixed.probg[:, ::5, b] = tab.probg[:, ::5, b], tab.probg[:, ::5, a]
+    p = P.base_params(6, 4, 5, photmax=photmax, nVar=2, fact_mesh=1.5, seed=a + b)
+    T = F.channel_field(p, 600.0, 1500.0, noise=0.02, seed=4)
+    o = O.Oracle(p, tab, T)
+    de32, de32d, _, _ = o.solve(O.all_cells(p))
+    o.close()
+    s = Solver(p, mixed)
+    s.set_fields([T])
+    s.solve(VARIANT_PLAIN)
+    assert np.array_equal(s.tallies(), de32.astype(np.float64))
+    s.solve(VARIANT_BATCHED)
+    assert np.abs(s.tallies() - de32d).max() <= 1e-12 * np.abs(de32d).max()
+    s.close()
+
+
+@pytest.mark.parametrize("nB", [513, 1024, 2000, 2048, 4095])
+@pytest.mark.parametrize("photmax", [100, 257])
+def test_high_digits(nB, photmax):
+    """bands repeated up to nB: nB nQ of 8208 to 65520 keys, high digits of 6
+    to 8 bits"""
+    a = synthetic_nb()
+    t = Tables(nB, a.nT, 16)
+    pick = np.arange(nB) % a.nB
+    for name in ("Tnb", "kP", "wq"):
+        getattr(t, name)[:] = getattr(a, name)
+    for name in ("wvl", "wvr", "wvc"):
+        getattr(t, name)[:] = getattr(a, name)[pick]
+    t.kavg[:] = np.random.default_rng(nB).permutation(nB) + 1.0
+    t.kq[:] = a.kq[pick]
+    t.prob[:] = ((np.arange(nB) + 1.0) / nB).astype(np.float32)
+    t.probg[:] = a.probg[:, pick]
+    p = P.base_params(6, 4, 5, photmax=photmax, nVar=2, fact_mesh=1.5, seed=nB)
+    p.nB = nB
+    solve_both(p, t, F.channel_field(p, 600.0, 1500.0, noise=0.02, seed=6))
