@@ -119,8 +119,6 @@ __device__ __forceinline__ SnapView snap_view(const DevSnap *snp) {
     v.bp = uni(snp->bp);
     v.xu_all = uni(snp->xu_all);
     v.P_all = uni(snp->P_all);
-    v.nxu = uni(snp->nxu);
-    v.npos = uni(snp->npos);
     return v;
 }
 
@@ -533,8 +531,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
             }
             __syncthreads();
         }
-        /* one back-edge: a unit may start and generate in the same iteration;
-         * an iteration with no live lane steps idle lanes only */
+        /* one back-edge: a unit may start and generate in the same iteration */
         {
             /* (c) bulk generation: every lane sets up one ray of the current unit */
             const int left = P - cur_h;
@@ -725,7 +722,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                 for (int g = 0; g < lev; ++g) xoff += llev[g].im + 1;
                 for (;;) {
                     const DevLevel L = llev[lev];
-                    march_ahead<TM, true>(cm, sv, L, r, e, tol, dacc, counter, nsteps, xul + xoff, L.maxs);
+                    march_ahead<TM>(cm, sv, L, r, e, tol, dacc, counter, nsteps, xul + xoff, L.maxs);
                     if (!(r.tra > tol) || lev == cm.grid_num - 1) break;
                     /* coarsen the indices for the next grid level */
                     r.ic = coarsen(r.ic, L.cr[0], L.cmul[0]);
@@ -744,7 +741,7 @@ __device__ __forceinline__ void batched_body(const DevCommon &cm, const DevSnap 
                 if (act == 0ull) break;
                 if (__popcll(act) > COOP_RAYS) {
                     if (active) {
-                        march_ahead<TM, true>(cm, sv, l0, r, e, tol, dacc, counter, nsteps, xul,
+                        march_ahead<TM>(cm, sv, l0, r, e, tol, dacc, counter, nsteps, xul,
                                               min(l0.maxs, counter + DRAIN_BLOCK));
                         if (!(r.tra > tol) || counter >= l0.maxs) {
                             finish_ray(cm, sl, seq, (int)(b.uh & 0xFFFFu), b.tid, (int)(b.uh >> 16), dacc, de);

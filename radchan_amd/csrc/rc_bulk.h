@@ -11,13 +11,13 @@
  *    and converts no index;
  *  - per axis the value of that index at which the ray has left the grid, so
  *    leaving is one comparison, made only in the branch of the axis crossed;
- *  - lanes without a live ray are masked off the step, so no load needs a
- *    bound;
+ *  - lanes without a live ray are masked off the step, and a live ray's
+ *    offsets are always a cell's or a wall entry's, so no load has a bound;
  *  - what happens once per ray (the dump tally, the finished ray's sums)
  *    waits until the lane's next pick-up, where it is done for all lanes
  *    that ended since.
  *
- * Every value is the one march_core and boundary compute, so the tallies
+ * Every value is the one march_step_thread computes, so the tallies
  * are the plain march's to the bit (but for the sign of a zero).
  *
  * Measured (march kernel, nVar 2, against the step that recomputed indices

@@ -168,7 +168,7 @@ struct rc_ctx {
     TableSet nbset;
     std::vector<Grid> grids;
     DevBuf xuall, x0, y0, z0;               /* x faces of every level, level g at xoff[g] */
-    int xoff[RC_MAXLEV] = {}, nxu = 0;
+    int xoff[RC_MAXLEV] = {};
     size_t poff[RC_MAXLEV] = {}, npos = 0;  /* level g's table positions at poff[g] */
     DevBuf cx[RC_MAXLEV], cy[RC_MAXLEV], cz[RC_MAXLEV];   /* cell centres per level */
     DevBuf spl;                             /* spline restriction scratch */
@@ -493,8 +493,6 @@ int push_snaps(rc_ctx *c) {
         d.Ibmax64 = S.Ibmax64; d.Ibmax_w64 = S.Ibmax_w64; d.Ibmax_e64 = S.Ibmax_e64;
         d.Tnb0d = (double)ts.Tnb[0];
         d.invdTd = 1.0 / (double)(ts.Tnb[1] - ts.Tnb[0]);
-        d.nxu = c->nxu;
-        d.npos = (int)c->npos;
         d.x0 = c->x0.as<float>(); d.y0 = c->y0.as<float>(); d.z0 = c->z0.as<float>();
         d.imax = p.imax; d.jmax = p.jmax; d.kmax = p.kmax; d.zstart = c->zstart;
         d.ncell = c->ncell; d.nsurf = c->nsurf;
@@ -712,7 +710,6 @@ rc_ctx *rc_create(const rc_params *pp) {
             upload(c->cz[g], c->grids[g].z, c->stream))
             return nullptr;
     }
-    c->nxu = (int)xuall.size();
     if (c->npos >= ((size_t)1 << 31)) { set_error("grid too large: table positions of all levels beyond 2^31"); return nullptr; }
     if (upload(c->xuall, xuall, c->stream)) return nullptr;
     if (upload(c->x0, c->grids[0].x, c->stream) || upload(c->y0, c->grids[0].y, c->stream) ||

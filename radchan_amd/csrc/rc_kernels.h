@@ -101,7 +101,6 @@ struct DevSnap {
     const float *T0;               /* ghost-padded input field            */
     const float *xu_all;           /* x faces of every level, level g at lev[g].xoff */
     const float *P_all;            /* table positions of every level, g at lev[g].poff */
-    int nxu, npos;                 /* their lengths                       */
     const float *x0, *y0, *z0;     /* level-0 cell centres                */
     /* the full-FP64 path (floatpoint 1): the temperatures behind P_all (same
      * layout), the weights in double and the table's temperature map */

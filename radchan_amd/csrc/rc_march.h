@@ -76,7 +76,6 @@ struct SnapView {
     const uint32_t *kp16;
     const float4 *bp;
     const float *xu_all, *P_all;
-    int nxu, npos;
 };
 
 /* k and Ib of table row `row` at row t with weight a */
@@ -251,22 +250,6 @@ __device__ __forceinline__ int boundary_move(const DevCommon &cm, const S &sn, c
     return RB_LOST;
 }
 
-/* the boundary condition with its tally: the wall emission tally ends the
- * ray at a wall; a lost ray ends with nothing */
-template <int TM = TAB_RT, class S>
-__device__ __forceinline__ void boundary(const DevCommon &cm, const S &sn, const DevLevel &L, Ray &r, const En &e,
-                                      float &de, int &status) {
-    float Bw = 0.f;
-    const int b = boundary_move<TM>(cm, sn, L, r, e, Bw);
-    if (b == RB_WALL) {
-        wall_hit(e, r, Bw, de);
-        status = RC_RAY_WALL;
-    } else if (b == RB_LOST) {
-        r.tra = 0.f;
-        status = RC_RAY_LOST;
-    }
-}
-
 /* The geometry of one march step (one iteration of march_ray's loop,
  * mc_gpu_noint.cu:252-654), given the x face the ray heads for
  * (fx = xu[ic - f0]): distances to the three candidate faces, the segment
@@ -297,34 +280,19 @@ __device__ __forceinline__ bool geo_move(const G &L, Ray &r, float fx, float &ds
            (uint32_t)(r.kc - 1) >= (uint32_t)L.km;
 }
 
-/* the linear index of the ray's cell on its level (clamped: a lane whose
- * state is stale reads in bounds) */
-__device__ __forceinline__ uint32_t cell_index(const DevLevel &L, const Ray &r) {
+/* The geometry of one march step of a live ray, `cell` the linear index of
+ * the cell that its segment crosses, on its level; `xul`: the level's x faces
+ * in LDS.  Both indices are in range for a ray inside the grid; the bounds
+ * keep any other in the level's arrays. */
+__device__ __forceinline__ bool geo_core(const DevLevel &L, Ray &r, uint32_t &cell, float &ds, const float *xul) {
+    const float fx = xul[min((uint32_t)(r.ic - r.f0), (uint32_t)L.im)];
     /* 24-bit products (full rate): the factors are below 2^24 for every
      * grid whose jm km and im are, and the product is the cell index */
-    return min((uint32_t)(r.ic - 1) + __umul24((uint32_t)L.im, (uint32_t)(r.jc - 1) +
+    cell = min((uint32_t)(r.ic - 1) + __umul24((uint32_t)L.im, (uint32_t)(r.jc - 1) +
                                                                   __umul24((uint32_t)L.jm, (uint32_t)(r.kc - 1))),
                (uint32_t)L.ncell - 1u);
-}
-
-/* geo_move, with `cell` the cell the segment crosses */
-__device__ __forceinline__ bool geo_core_fx(const DevLevel &L, Ray &r, float fx, uint32_t &cell, float &ds) {
-    cell = cell_index(L, r);
     bool xa, ya;
     return geo_move(L, r, fx, ds, xa, ya);
-}
-
-/* geo_core_fx with the x face looked up: in global memory, or with XL in
- * an LDS copy */
-template <bool XL = false>
-__device__ __forceinline__ bool geo_core(const DevLevel &L, Ray &r, uint32_t &cell, float &ds,
-                                         const float *xul = nullptr) {
-    /* both indices are in range for a ray inside the grid; the bounds only
-     * matter to a lane whose state is stale (the batched kernel steps idle
-     * lanes too and discards what they compute) */
-    const uint32_t ix = min((uint32_t)(r.ic - r.f0), (uint32_t)L.im);
-    const float fx = XL ? xul[ix] : gld32(L.xu, ix);
-    return geo_core_fx(L, r, fx, cell, ds);
 }
 
 /* The absorption of one step with optical depth -x (x = -K ds): attenuation
@@ -350,21 +318,6 @@ __device__ __forceinline__ void phys_core(float K, float B, float ds, const En &
     phys_core_x(-(K * ds), B, e, tol, tra, de, status);
 }
 
-/* one march step: geometry, then the absorption at the crossed cell's
- * table position (table interpolation, FP32).  Select-based, no branch;
- * returns whether an index left the grid. */
-template <int TM = TAB_RT, class S>
-__device__ __forceinline__ bool march_core(const DevCommon &cm, const S &sn, const DevLevel &L, Ray &r,
-                                           const En &e, float tol, float &de, int &status) {
-    uint32_t cell;
-    float ds;
-    const bool out = geo_core(L, r, cell, ds);
-    float K, B;
-    kb_pos<TM>(sn, e.row, e.rank, cm.nT, gld32(L.P, cell), K, B);
-    phys_core(K, B, ds, e, tol, r.tra, de, status);
-    return out;
-}
-
 /* the index ic on the next level, (ic + r - 1) / r (mc_gpu_noint.cu:215-223),
  * by the level's multiplier */
 __device__ __forceinline__ int coarsen(int ic, int r, uint32_t m) {
@@ -377,14 +330,14 @@ __device__ __forceinline__ int coarsen(int ic, int r, uint32_t m) {
  * reaches `limit` (at most the level's step cap L.maxs), with the geometry
  * two steps ahead of the absorption: the temperature of step i+2 and the
  * table entries of step i+1 are loaded while step i is absorbed.  The
- * arithmetic of every step is that of march_step, so the tally,
+ * arithmetic of every step is that of march_step_thread, so the tally,
  * transmissivity and step count are bit-identical; only a dumped ray's
  * final position differs (the geometry ran ahead of it).  A ray stopped by
  * the limit has taken exactly its steps up to the limit, so the march can
- * resume from it.  Expects a live ray below the limit.  With XL the
- * level's x faces come from an LDS copy (xul), so that the geometry never
- * waits on the vector-memory counter behind the prefetched loads. */
-template <int TM = TAB_RT, bool XL = false, class S>
+ * resume from it.  Expects a live ray below the limit.  The level's x faces
+ * come from an LDS copy (xul), so that the geometry never waits on the
+ * vector-memory counter behind the prefetched loads. */
+template <int TM = TAB_RT, class S>
 __device__ __forceinline__ void march_ahead(const DevCommon &cm, const S &sn, const DevLevel &L, Ray &r,
                                             const En &e, float tol, float &de, int &counter, int &nsteps,
                                             const float *xul, int limit) {
@@ -394,7 +347,7 @@ __device__ __forceinline__ void march_ahead(const DevCommon &cm, const S &sn, co
     uint32_t c0;
     float d0, w0;
     int b0 = RB_ON;
-    if (geo_core<XL>(L, r, c0, d0, xul)) b0 = boundary_move<TM>(cm, sn, L, r, e, w0);
+    if (geo_core(L, r, c0, d0, xul)) b0 = boundary_move<TM>(cm, sn, L, r, e, w0);
     KbRaw k0 = kb_fetch<TM>(sn, e.row, e.rank, nT, gld32(L.P, c0));
     /* step i+1 */
     /* The loads are issued on every path (cell 0 for a step not taken,
@@ -406,7 +359,7 @@ __device__ __forceinline__ void march_ahead(const DevCommon &cm, const S &sn, co
     float d1, w1;
     int b1 = RB_ON;
     if (h1)
-        if (geo_core<XL>(L, r, c1, d1, xul)) b1 = boundary_move<TM>(cm, sn, L, r, e, w1);
+        if (geo_core(L, r, c1, d1, xul)) b1 = boundary_move<TM>(cm, sn, L, r, e, w1);
     float p1 = gld32(L.P, c1);
     for (;;) {
         /* step i+2: geometry and temperature */
@@ -415,7 +368,7 @@ __device__ __forceinline__ void march_ahead(const DevCommon &cm, const S &sn, co
         float d2, w2;
         int b2 = RB_ON;
         if (h2)
-            if (geo_core<XL>(L, r, c2, d2, xul)) b2 = boundary_move<TM>(cm, sn, L, r, e, w2);
+            if (geo_core(L, r, c2, d2, xul)) b2 = boundary_move<TM>(cm, sn, L, r, e, w2);
         const float p2 = gld32(L.P, c2);
         /* step i+1: table entries */
         const KbRaw k1 = kb_fetch<TM>(sn, e.row, e.rank, nT, p1);
@@ -458,7 +411,7 @@ __device__ __forceinline__ float quad_lane(float x) {
  * transmissivity is carried through the steps in order (lane s receives
  * the value before its step), the step that ends the ray found by a
  * ballot, and the tally terms, computed per lane, summed in step order.
- * Every product and sum is the one march_step makes, on the same values
+ * Every product and sum is the one march_step_thread makes, on the same values
  * and in the same order, so the tally, transmissivity and step count are
  * bit-identical to it.  Returns at the ray's end or at the level's step
  * cap; expects a live ray under the cap.  `xul`: the level's x faces in
@@ -612,15 +565,8 @@ __device__ __forceinline__ void march_coop(const DevCommon &cm, const S &sn, con
     }
 }
 
-/* march_core, then the boundary condition of the face crossed, if any */
-template <int TM = TAB_RT, class S>
-__device__ __forceinline__ void march_step(const DevCommon &cm, const S &sn, const DevLevel &L, Ray &r,
-                                           const En &e, float tol, float &de, int &status) {
-    if (march_core<TM>(cm, sn, L, r, e, tol, de, status)) boundary<TM>(cm, sn, L, r, e, de, status);
-}
-
 /* The boundary condition of the face crossed, as a branch over the face:
- * the same outcome and tally as boundary(), in the form a thread that
+ * boundary_move's outcome with its tally, in the form a thread that
  * marches its own ray (plain variant, traced rays) runs fastest -- its
  * lanes cross faces at steps of their own, so the face code is read only
  * where one is crossed. */
@@ -663,9 +609,9 @@ __device__ __forceinline__ void boundary_thread(const DevCommon &cm, const DevSn
     }
 }
 
-/* one march step of a thread that marches its own ray: march_core's
- * arithmetic with the table-position load issued as soon as the cell index
- * is known, then boundary_thread */
+/* one march step of a thread that marches its own ray (one iteration of
+ * march_ray's loop): geometry, with the table-position load issued as soon as
+ * the cell index is known, absorption, then boundary_thread */
 __device__ __forceinline__ void march_step_thread(const DevCommon &cm, const DevSnap &sn, const DevLevel &L, Ray &r,
                                                   const En &e, float tol, float &de, int &status) {
     const float fx = gld32(L.xu, min((uint32_t)(r.ic - r.f0), (uint32_t)L.im));
