@@ -864,23 +864,22 @@ void launch_zero(hipStream_t st, double *p, size_t n) {
 }
 
 /* workgroups per CU by default: 32 on a single grid, 20 on several levels
- * (what the autotuner picks on 256x128x256 and 192x128x192) */
+ * (the autotuner's 20 to 40 are within 1 % of each other) */
 static int default_wg_per_cu(const DevCommon &cm, int wg_per_cu) {
     return wg_per_cu > 0 ? wg_per_cu : (cm.grid_num > 1 ? 20 : 32);
 }
 
 /* Defaults of the schedule (a refill mode < 0, a threshold or steps per
- * iteration <= 0).  Single grid: refills at 8 idle lanes (4: 2 % slower at
- * 256x128x256), also between the steps, 6 steps per iteration: within 1 % of the autotuner's pick at
- * 256x128x256 (8 steps) and of the best at 64^3, where rays of 6 steps end
- * faster than the one round of 64 new rays per iteration replaces them at
- * 8 steps (0.60 of the lanes active, 10 % slower).
- * Several levels: refills at 4 idle lanes once per iteration and as
- * many steps per iteration as the finest level's step cap, so that the
- * rays a wavefront picks up together reach that cap, and hand off to the
- * next level, on the same step: one pass through the hand-off serves all
- * of them (param.h's maxs 5 on its 406x576x2304 share: 6.27 s against
- * 6.60 s with 4 steps and refills between them). */
+ * iteration <= 0).  Single grid: refills at 8 idle lanes, also between the
+ * steps, 6 steps per iteration.  Several levels: refills at 4 idle lanes once
+ * per iteration and as many steps per iteration as the finest level's step
+ * cap, so that the rays a wavefront picks up together reach that cap, and
+ * hand off to the next level, on the same step: one pass through the hand-off
+ * serves all of them.  March by default against the autotuner's best: 64^3,
+ * 200 rays 7.36 and 7.12 ms (3 steps, refills once per iteration),
+ * 256x128x256 177.3 and 176.9 (4 steps, likewise), 192x128x192 at three
+ * levels 49.03 and 49.05, param.h's settings on 28x96x128 89.6 and 89.6
+ * (its own choice: the default's steps). */
 void batched_schedule(const DevCommon &cm, int &wg_per_cu, int &threshold, int &spi, int &refill) {
     const bool mg = cm.grid_num > 1;
     if (refill < 0) refill = mg ? 0 : 1;

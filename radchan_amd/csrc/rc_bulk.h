@@ -22,9 +22,12 @@
  *
  * Measured (march kernel, nVar 2, against the step that recomputed indices
  * and addresses and stepped idle lanes too): 256x128x256, 360 bands, photmax
- * 100 200.1 -> 195.6 ms (its gathers keep the texture-address units 0.83
- * busy); four snapshots of 64x96x64 and 110x62x90 with BF16 tables
- * 51.4 -> 38 ms; param.h's settings on 28x96x128, one run 106.2 -> 97.2 ms.
+ * 100 200.1 -> 195.6 ms; four snapshots of 64x96x64 and 110x62x90 with BF16
+ * tables 51.4 -> 38 ms; param.h's settings on 28x96x128, one run 106.2 -> 97.2
+ * ms; with the ray generation, the queue and the exponent as they are now
+ * 176.4, 34.5 and 89.8 ms.  A step's straight path is 86 vector instructions.
+ * At 256x128x256 the gathers keep the texture-address units 0.88 busy, with
+ * the vector issue at 0.75; at three levels (192x128x192) the issue is full.
  */
 #ifndef RC_BULK_H
 #define RC_BULK_H

@@ -263,8 +263,9 @@ __device__ __forceinline__ double gg_at(int j, const uint16_t *RB, const double 
     return lo < r1 ? G[lo] : 1.0;
 }
 
-/* up to 1024 pairs: 7 workgroups per CU (72 registers, a few spilled), 1.03 ms at 47 580 spectra of 1000 points; unbounded (82
- * registers, 5 workgroups) 1.19, 6 1.06, 8 (64 registers) 1.11 */
+/* up to 1024 pairs: 7 workgroups per CU (72 registers and 9 or 10 spilled, 36 bytes a thread and 0.44 GB of writes at
+ * 47 580 spectra of 1000 points), 1.03 ms there; unbounded (82 registers, 5 workgroups) 1.19, 6 1.06, 8 (64
+ * registers) 1.11 */
 template <int R>
 __global__ __launch_bounds__(CK_THREADS, R <= 4 ? 7 : 1) void k_ckdist(CkArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];

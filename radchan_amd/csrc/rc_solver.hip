@@ -528,9 +528,13 @@ __device__ __forceinline__ void coarsen64(const DevSnap &sn, int g, int &ic, int
  * step) and the rest the last rays: a lone lane's step takes about 3000
  * clocks, coop64's 400 (15.3 ms per run without it).  REFILL64 4 to 16 and
  * STEPS64 1 to 4 are within 5 %; COOP64 4 to 16 within 1 %; 3 wavefronts per
- * SIMD instead of 4 (128 registers, a few spills) 2 % slower; stopping the
- * wavefront for a ray of over 1000 steps to march it together at once, the
- * same. */
+ * SIMD instead of 4 (128 registers, 10 or 11 of them spilled, 46 with several
+ * levels) 2 % slower; stopping the wavefront for a ray of over 1000 steps to
+ * march it together at once, the same.  Thread per cell -> now elsewhere: 64^3,
+ * 200 rays, 8 runs 201 -> 43 ms; 192x128x192, 100 rays, one run, one level
+ * 319 -> 107 (two launches, the tallies' 2 GiB), three levels with walls
+ * 108 -> 101, 8 runs 857 -> 797; param.h's settings on 28x96x128, 2 runs,
+ * whose rays end after 3.4 steps and fill the lanes either way, 601 -> 578. */
 constexpr int REFILL64 = 8, STEPS64 = 2;
 static_assert(COOP64 * sizeof(Drain64) + sizeof(Chain64) <= sizeof(Rec64), "the drain's LDS");
 
