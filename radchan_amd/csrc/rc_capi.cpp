@@ -73,6 +73,7 @@ struct DevBuf {
         if (n == 0) n = 16;
         if (hipMalloc(&p, n) != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();    /* reported here, not by the next launch's check */
             set_error("device allocation of " + std::to_string(n) + " bytes failed");
             return -11;
         }
@@ -967,7 +968,6 @@ int rc_run(rc_ctx *c, int variant) {
             const size_t nr = (size_t)std::max(c->ncell, p.calcwalls == 1 ? 2 * c->nsurf : 0) * p.photmax;
             c->runs64 = fp64_scratch(c->keys, c->ray64, keys ? nk : 0, nr, (size_t)p.photmax, p.nVar);
             if (!c->runs64) return -11;
-            (void)hipGetLastError();    /* of the sizes there was no memory for */
         } else if (keys) {
             if (int e = c->keys.ensure(nk * 2)) return e;
         }
@@ -985,7 +985,6 @@ int rc_run(rc_ctx *c, int variant) {
                                         c->srt_refused);
         if (c->srtk.p != old || beside != c->srt_beside) c->drop_graph();
         if (beside < 0) return -11;
-        (void)hipGetLastError();        /* of a size there was no memory for */
         c->srt_beside = beside;
     }
     if (variant == RC_VARIANT_BATCHED && c->reduction == 1) {
@@ -1449,7 +1448,6 @@ int rc_group_run(rc_group *g) {
     const size_t nf = batched_srt_keys(cm, cells, g->wg_per_cu);
     const int beside = sort_scratch(g->srtk, nf, walls ? batched_srt_keys(cm, wcells, g->wg_per_cu) : 0, g->srt_refused);
     if (beside < 0) return -11;
-    (void)hipGetLastError();            /* of a size there was no memory for */
     cm.srt_keys = g->srtk.as<uint16_t>();
     DevCommon cw = cm;
     if (beside) cw.srt_keys += nf;
